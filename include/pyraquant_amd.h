@@ -55,10 +55,12 @@ extern "C" {
 #define PQ_EDTYPE (-4)  /* unsupported dtype code                         -> Python ValueError     */
 #define PQ_ELAUNCH (-5) /* HIP runtime error at launch                    -> Python RuntimeError   */
 
-/* element type codes of the 16-bit floating operands (and, for pq_int8_gemm_packed's output, raw int32) */
+/* element type codes of the 16-bit floating operands (and, for pq_int8_gemm_packed's output, raw int32; for
+ * pq_convert_weight's input, fp32) */
 #define PQ_BF16 0
 #define PQ_F16 1
 #define PQ_I32 2
+#define PQ_F32 3
 
 /* flag OR'ed into pq_int8_gemm_packed's out_dtype: accumulate into c instead of overwriting it,
  * c[o, n] = round(c[o, n] + round(y)) (two 16-bit roundings, as torch adds two 16-bit tensors) */
@@ -99,6 +101,16 @@ int pq_quant_rows(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t 
  */
 int pq_quant_weight(const float* w, int64_t N, int64_t K, int64_t ldw, int64_t group, int8_t* q, float* s,
                     hipStream_t stream);
+
+/*
+ * pq_quant_weight for a weight of any of the types models hold (dtype PQ_BF16, PQ_F16 or PQ_F32; 16-bit values widen
+ * to fp32 exactly, so the codes and scales are those of the widened weight), with the codes also written in the packed
+ * K64 layout (qp [N * K], as pq_pack_k64 writes them; K % 64 == 0, N % 16 == 0, q and qp 16-byte aligned) unless qp is
+ * NULL. One pass over the weight where its rows are 16-byte aligned, K % 8 == 0 and group is 0 or 32. Replaces the
+ * conversion of `Int8Linear.__init__` (deploy/int8_exec.py:350-359).
+ */
+int pq_convert_weight(const void* w, int32_t dtype, int64_t N, int64_t K, int64_t ldw, int64_t group, int8_t* q, float* s,
+                      int8_t* qp, hipStream_t stream);
 
 /*
  * Low-rank down-projection t = x[rows] @ lr_A, fp32 accumulation, rounded to the 16-bit type of x.

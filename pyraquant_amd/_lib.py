@@ -15,7 +15,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime first, so the library bin
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libpqint8.so")
 
 PQ_OK, PQ_EINVAL, PQ_ESHAPE, PQ_EALIGN, PQ_EDTYPE, PQ_ELAUNCH = 0, -1, -2, -3, -4, -5
-PQ_BF16, PQ_F16, PQ_I32 = 0, 1, 2
+PQ_BF16, PQ_F16, PQ_I32, PQ_F32 = 0, 1, 2, 3
 PQ_ACCUMULATE = 0x100   # OR'ed into pq_int8_gemm_packed's out_dtype
 ABI_VERSION = 3
 
@@ -25,6 +25,7 @@ EXPORTS = (
     "pq_last_error",
     "pq_quant_rows",
     "pq_quant_weight",
+    "pq_convert_weight",
     "pq_lowrank_down",
     "pq_int8_gemm",
     "pq_int8_gemm_i32",
@@ -54,6 +55,7 @@ _SIGNATURES = {
     "pq_last_error": ([], ctypes.c_char_p),
     "pq_quant_rows": ([_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _p, _p], ctypes.c_int),
     "pq_quant_weight": ([_p, _i64, _i64, _i64, _i64, _p, _p, _p], ctypes.c_int),
+    "pq_convert_weight": ([_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _p, _p], ctypes.c_int),
     "pq_lowrank_down": ([_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _i64, _p, _i64, _p], ctypes.c_int),
     "pq_int8_gemm": ([_p, _i64, _p, _i64, _p, _p, _i64, _p, _p, _i64, _p, _i64, _i32, _p, _i64, _i32, _p, _i64,
                       _i64, _i64, _i64, _p, _p], ctypes.c_int),

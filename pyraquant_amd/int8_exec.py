@@ -375,22 +375,34 @@ def int8_linear_2d(x2: torch.Tensor, w_int8: torch.Tensor, w_scale: torch.Tensor
 
 
 # --------------------------------------------------------------------------- weight quantization
-def quantize_weight(w: torch.Tensor, group_size: int = 0) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Weight RTN on the GPU (pq_quant_weight), fp32 math with IEEE divisions.
-    group_size 0: per output channel, s [N] (deploy/int8_exec.py:355-357).
-    group_size g: qdq_weight(w, 8, g) codes and scales, s [N, K/g] (pyraquant/quantizers_weight.py:96-109)."""
+_WEIGHT_DTYPES = {torch.bfloat16: _lib.PQ_BF16, torch.float16: _lib.PQ_F16, torch.float32: _lib.PQ_F32}
+
+
+def _convert_weight(w: torch.Tensor, group_size: int, pack: bool):
+    """(codes [N, K], scales, codes in the packed K64 layout or None), pq_convert_weight."""
     assert w.dim() == 2 and w.is_cuda, "weight quantization runs on the GPU (move the Linear to the device first)"
-    wf = w.detach().float()
-    if wf.stride(1) != 1:
-        wf = wf.contiguous()
-    N, K = wf.shape
+    wk = w.detach()
+    if wk.dtype not in _WEIGHT_DTYPES:
+        wk = wk.float()
+    if wk.stride(1) != 1:
+        wk = wk.contiguous()
+    N, K = wk.shape
     if group_size:
         assert K % group_size == 0, (K, group_size)
     q = torch.empty((N, K), dtype=torch.int8, device=w.device)
     s = torch.empty((N, K // group_size) if group_size else (N,), dtype=torch.float32, device=w.device)
+    qp = torch.empty((packed_rows(N) * K,), dtype=torch.int8, device=w.device) if pack else None
     L = _lib.load()
-    _lib.check(L.pq_quant_weight(_lib.ptr(wf), N, K, wf.stride(0), group_size, _lib.ptr(q), _lib.ptr(s),
-                                 _lib.stream_of(w.device)), "quant_weight")
+    _lib.check(L.pq_convert_weight(_lib.ptr(wk), _WEIGHT_DTYPES[wk.dtype], N, K, wk.stride(0), group_size, _lib.ptr(q),
+                                   _lib.ptr(s), _lib.ptr(qp), _lib.stream_of(w.device)), "quant_weight")
+    return q, s, qp
+
+
+def quantize_weight(w: torch.Tensor, group_size: int = 0) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Weight RTN on the GPU (pq_convert_weight), fp32 math with IEEE divisions.
+    group_size 0: per output channel, s [N] (deploy/int8_exec.py:355-357).
+    group_size g: qdq_weight(w, 8, g) codes and scales, s [N, K/g] (pyraquant/quantizers_weight.py:96-109)."""
+    q, s, _ = _convert_weight(w, group_size, False)
     return q, s
 
 
@@ -429,14 +441,15 @@ class Int8Linear(nn.Module):
         w = lin.weight.detach()
         if device is not None:
             w = w.to(device, non_blocking=False)
-        q, s = quantize_weight(w, group_size)
+        # layers whose shape the packed GEMM takes (per-channel and group-32) run on the packed K64 path
+        pack = w.dim() == 2 and w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0
+        q, s, packed = _convert_weight(w, group_size, pack)
         self.group_size = int(group_size)
         self.register_buffer("weight_int8", q)
         self.register_buffer("w_scale", s)
         N, K = q.shape
-        # layers whose shape the packed GEMM takes (per-channel and group-32) run on the packed K64 path
-        if K % 64 == 0 and N % 64 == 0:
-            self.register_buffer("weight_packed", pack_k64(q))
+        if pack:
+            self.register_buffer("weight_packed", packed)
         else:
             self.weight_packed = None
         if group_size:

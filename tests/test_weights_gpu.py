@@ -249,3 +249,35 @@ def test_accumulate_scatter_and_group32(cuda):
         expect[ori.long()] = expect[ori.long()] + y
         q(x, row_idx=ri, out=canvas, out_row_idx=ori, accumulate=True)
         assert torch.equal(canvas, expect), group
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("K,group", [(64, 0), (520, 0), (1024, 0), (3072, 0), (6208, 0), (12288, 0), (15360, 0), (16448, 0),
+                                     (64, 32), (640, 32), (2080, 32), (96, 48)])
+def test_convert_weight_one_pass(cuda, dtype, K, group):
+    """pq_convert_weight's vectorised kernels (register rows at every chunk count, two sweeps, groups of 32) against
+    its element-by-element kernel, which a weight at an odd element offset takes, and against the oracle: the same
+    codes and scales bit for bit, also for ties, a zero row, NaN and infinite weights; the packed codes are
+    pack_k64's."""
+    from oracle import oracle as O
+    from pyraquant_amd import int8_exec as E
+
+    N = 80
+    g = torch.Generator().manual_seed(K + group)
+    w = (torch.randn(N, K, generator=g) * 0.02).to(dtype)
+    w[1] = 0
+    w[2, 0], w[2, 1:] = 127.0, torch.arange(K - 1).remainder(127).to(dtype) + 0.5   # scale 1: ties
+    w[3] *= 1e-6
+    finite = w.clone()
+    w[4, 5], w[5, 7], w[6] = float("nan"), float("inf"), float("nan")
+    for vals in (finite, w):
+        wide = torch.zeros(N, K + 8, dtype=dtype, device=cuda)
+        wide[:, 1:K + 1] = vals.to(cuda)
+        q, s, qp = E._convert_weight(vals.to(cuda), group, K % 64 == 0)
+        q1, s1 = E.quantize_weight(wide[:, 1:K + 1], group)
+        assert torch.equal(q, q1) and torch.equal(s, s1)
+        if qp is not None:
+            assert torch.equal(qp, E.pack_k64(q1))
+    q, s = E.quantize_weight(finite.to(cuda), group)
+    qo, so = O.quant_weight(finite.float().numpy(), group)
+    assert (q.cpu().numpy() == qo).all() and (s.cpu().numpy() == so).all()
