@@ -8,12 +8,14 @@
 // of 8 elements per lane), so x is read from HBM exactly once. The absmax is a packed-u16 max over the
 // magnitude bits (monotonic in |x| for finite 16-bit floats) and a wave reduction.
 //
-// Exact codes without one IEEE division per element: with c = fl(1/s) and v = x * c (exact product),
-// |v - x / s| <= |x| |c - 1/s| <= 127 * 2^-24 and |x / s - fl(x / s)| <= 127 * 2^-24, so |v - fl(x / s)| < 1.6e-5:
-// whenever v is farther than kTieMargin from every half-integer, rint(v) == rint(fl(x / s)). One fma gives
-// m = fl(v + 1.5 * 2^23) = 1.5 * 2^23 + rint(v) (round to nearest even; |v| < 2^22), whose low byte is the int8
-// code, and a second gives the residual fl(v - rint(v)), whose largest magnitude over 8 elements is tested once.
-// Chunks with an element within the margin (about one element in 10^4) redo it with the correctly rounded division.
+// Exact codes without one IEEE division per element and without a branch: with c = fl(1/s),
+//   q0 = fl(x c); r = fma(-q0, s, x) (the remainder of q0, exact); q = fma(r, c, q0)
+// is the Newton step that ends a correctly rounded division, and rint(q) == rint(fl(x / s)) for every row maximum a and
+// every |x| <= a of both 16-bit types: the result depends on the two mantissas and the exponent difference alone, and
+// all of those pairs (and the floor s = fl(1e-8) / 127) have been compared. q + 1.5 * 2^23 holds the rounded code in its
+// low byte (round to nearest even; |q| < 2^22). Four instructions per element. A test for near ties with the division
+// beside it was as many, and its code, repeated for every chunk of a row, was what bound the kernels: 1.7 KB per
+// chunk, up to 84 KB in a kernel against the 64 KB instruction cache that two CUs share.
 #include "pq_common.h"
 
 #include <algorithm>
@@ -26,7 +28,7 @@ namespace pq {
 namespace {
 
 constexpr float kMagic = 12582912.0f;        // 1.5 * 2^23: x + kMagic rounds x to an integer (|x| < 2^22)
-constexpr float kTieMargin = 6.0e-5f;        // > 1.6e-5 error bound of v, see the header comment
+constexpr float kTieMargin = 6.0e-5f;        // weight_codes8: > 1.6e-5, the error bound of x fl(1/s) against fl(x / s)
 constexpr float kNearHalf = 0.5f - kTieMargin;
 
 // Code of one element: returns kMagic + q as fp32 (its low byte is the int8 code q).
@@ -43,25 +45,15 @@ __device__ __forceinline__ uint32_t low_bytes4(float m0, float m1, float m2, flo
   return __builtin_amdgcn_perm(b, a, 0x05040100u);
 }
 
-// Quantize 8 elements held in one 16-byte chunk; returns 8 int8 codes packed in a uint2.
+// Quantize 8 elements held in one 16-byte chunk; returns 8 int8 codes packed in a uint2 (see the header comment).
 template <int DT>
 __device__ __forceinline__ v2u quant_chunk(v4u v, float s, float rc) {
-  float f[8];
-  f[0] = lo16_to_f32<DT>(v.x); f[1] = hi16_to_f32<DT>(v.x);
-  f[2] = lo16_to_f32<DT>(v.y); f[3] = hi16_to_f32<DT>(v.y);
-  f[4] = lo16_to_f32<DT>(v.z); f[5] = hi16_to_f32<DT>(v.z);
-  f[6] = lo16_to_f32<DT>(v.w); f[7] = hi16_to_f32<DT>(v.w);
   float m[8];
-  float d = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    m[i] = __builtin_fmaf(f[i], rc, kMagic);
-    d = fmaxf(d, fabsf(__builtin_fmaf(f[i], rc, -(m[i] - kMagic))));
-  }
-  if (__builtin_expect(d > kNearHalf, 0)) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (fabsf(__builtin_fmaf(f[i], rc, -(m[i] - kMagic))) > kNearHalf) m[i] = code_exact(f[i], s);
+    const float f = i & 1 ? hi16_to_f32<DT>(v[i >> 1]) : lo16_to_f32<DT>(v[i >> 1]);
+    const float q0 = f * rc;
+    m[i] = __builtin_fmaf(__builtin_fmaf(-q0, s, f), rc, q0) + kMagic;
   }
   return v2u{low_bytes4(m[0], m[1], m[2], m[3]), low_bytes4(m[4], m[5], m[6], m[7])};
 }
@@ -328,8 +320,10 @@ __device__ __forceinline__ float absmax8(const float (&f)[8], float a) {
   for (int e = 0; e < 8; ++e) a = fmaxf(a, fabsf(f[e]));   // (a NaN element does not count, as in the scalar kernel)
   return a;
 }
-// The codes of 8 weights: quant_chunk's two fmas per element (their error bound holds for any fp32 input). Elements
-// near a tie, and those whose test is not a number (a NaN weight, or an infinite scale), take the division.
+// The codes of 8 weights of any fp32 value: with c = fl(1/s) and v = x c (exact product), |v - x / s| <= 127 * 2^-24 and
+// |x / s - fl(x / s)| <= 127 * 2^-24, so wherever v is farther than kTieMargin from every half-integer,
+// rint(v) == rint(fl(x / s)). One fma rounds v, a second gives its residual. Chunks with an element near a tie, or one
+// whose residual is not a number (a NaN weight, or an infinite scale), take the division.
 __device__ __forceinline__ v2u weight_codes8(const float (&f)[8], float s, float rc) {
   float m[8];
   bool far = true;
@@ -789,7 +783,8 @@ __global__ __launch_bounds__(256) void pack_lowrank_l1t_kernel(const v4u* __rest
 // Ordering: the L1^T DMA of slab e + 1 is issued after barrier e, when every wave has read that buffer's previous slab
 // (e - 1); it must land before barrier e + 1, and the only vector-memory instructions issued after it are slab e + 1's
 // RPW code stores and RPW next-batch loads, hence vmcnt(2 RPW) there (vector-memory instructions retire in issue
-// order).
+// order). The slab is straight-line code, so scheduling fences hold the DMA, those stores and loads, and the wait in
+// that order.
 // Past the last batch the next-batch loads read this batch's rows again (discarded), which keeps that count exact.
 constexpr int kWideWaves = 8;                 // waves per workgroup, two rows each: batches of 16 rows
 constexpr int kWideSlab = 512;                // K elements per slab
@@ -881,6 +876,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
       live[rho] = src_of(bn < nbatch ? bn : b, rho) >= 0;   // the batch whose loads xn starts
     }
     dma_l(0);   // lands before slab 0's barrier: only that slab's code stores and next-batch loads come after it
+    __builtin_amdgcn_sched_barrier(0);   // (and none of them before it: the vmcnt count below rests on the order)
     float sc[RPW], rc[RPW];
 #pragma unroll
     for (int rho = 0; rho < RPW; ++rho) {
@@ -921,12 +917,14 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
       // chunk e of the next batch into the registers just freed
 #pragma unroll
       for (int rho = 0; rho < RPW; ++rho) v[rho][e] = __builtin_nontemporal_load(xn[rho] + e * 64 + lane);
+      __builtin_amdgcn_sched_barrier(0);   // the slab's stores and loads stay between the DMA and this wait
       wait_vmcnt<2 * RPW>();   // this wave's DMA of L1^T slab e has landed (RPW stores, RPW loads after it)
       __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave's x slab writes are done
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_barrier();         // both slabs complete; every wave is done with slab e - 1
       __builtin_amdgcn_sched_barrier(0);
       if (e + 1 < NCH) dma_l(e + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < KW / 32; ++ks) {
         const int kk = wave * KW + ks * 32 + kg * 8;   // K offset inside the slab

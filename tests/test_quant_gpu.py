@@ -163,3 +163,35 @@ def test_linear_golden_fixture(cuda):
     ylr = E.int8_gemm_lr(q, s, wq, ws, b, t, l2.to(cuda), torch.bfloat16)
     mx, mean = rel_errors(ylr.float().cpu().numpy(), f["y_lr_f64"])
     assert mx <= MAX_REL and mean <= MEAN_REL, (mx, mean)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_quant_rows_every_mantissa_pair(oracle, cuda, dtype):
+    """Codes come from a branch-free Newton step, whose rounding depends on the row maximum's and the element's
+    mantissas and their exponent difference alone: every maximum (all 128 mantissas in bf16; every fifth of the 1024 in
+    fp16) against every element mantissa at exponent differences 0 .. 9 (below that every code is 0), both signs,
+    against the oracle bit for bit, in the packed and the row-major kernel."""
+    from pyraquant_amd import int8_exec as E
+
+    bf = dtype == torch.bfloat16
+    n, step, base = (128, 1, 0x3F80) if bf else (1024, 5, 0x4C00)
+    maxima = torch.arange(0, n, step) + base
+    elems = (torch.arange(-9 * n, n) + base).to(torch.int16)
+    elems = torch.cat([elems, elems | torch.tensor(-32768, dtype=torch.int16)])
+    rows = []
+    for a in maxima.tolist():
+        keep = torch.where((elems & 0x7FFF) <= a, elems, torch.zeros_like(elems))
+        keep[0] = a
+        rows.append(keep)
+    x = torch.stack(rows).view(dtype)
+    x = torch.nn.functional.pad(x, (0, (-x.shape[1]) % 64))
+    for r0 in range(0, x.shape[0], 64):
+        part = x[r0:r0 + 64].contiguous()
+        for c0 in range(0, part.shape[1], 8192):   # (the vectorised kernels take rows up to 16384)
+            xc = part[:, c0:c0 + 8192].clone()
+            xc[:, 0] = part[:, 0]
+            q, s = E.quant_rows(xc.to(cuda))
+            qo, so = oracle.quant_rows(bits(xc), dcode(dtype))
+            assert (q.cpu().numpy() == qo).all() and (s.cpu().numpy() == so).all()
+            qp, _ = E.quant_rows_packed(xc.to(cuda))
+            assert torch.equal(qp, E.pack_k64(q))
