@@ -79,13 +79,25 @@ __device__ __forceinline__ float absmax_from_bits(uint32_t mag16) {
   return lo16_to_f32<DT>(mag16);
 }
 
+constexpr int kMaxParts = 16;   // partial sums per row of t
+
+// Where partial sum p of t[m, r] waits in the packed code buffer (lowrank_partial_kernel -> quant_rows_vec_kernel): row
+// m owns 64 bytes of each of its KT blocks of 1 KB, and partial p (32 floats) takes the row's bytes of blocks 2 p and
+// 2 p + 1, so the wave that quantizes the row is the only one to read them and to overwrite them.
+__device__ __forceinline__ int64_t lr_part_offset(int64_t m, int p, int r, int KT) {
+  return ((m >> 4) * KT + 2 * p + (r >> 4)) * 1024 + (m & 15) * 64 + (r & 15) * 4;
+}
+
 // Vectorised quantizer: one wave per row, CH 16-byte chunks per lane, 4 rows per 256-thread block.
 // PACKED: codes go to the packed K64 layout (8-byte stores at k64_offset), and the waves of the padding rows
 // M .. 16 * ceil(M / 16) - 1 write zeros there. A gathered source row outside [0, x_rows) reads as zeros.
-template <int DT, int CH, bool PACKED>
+// PARTS: row m's bytes of q hold `parts` partial sums of its t (lowrank_partial_kernel) on entry: the row's wave adds
+// them in fp32, (p0 + p2 + ..) + (p1 + p3 + ..), and stores t before its codes take the bytes.
+template <int DT, int CH, bool PACKED, bool PARTS = false>
 __global__ __launch_bounds__(256) void quant_rows_vec_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int K, int64_t M, const int32_t* __restrict__ row_idx,
-    int8_t* __restrict__ q, float* __restrict__ s, int64_t x_rows, int32_t* __restrict__ zero9) {
+    int8_t* __restrict__ q, float* __restrict__ s, int64_t x_rows, int32_t* __restrict__ zero9, int parts,
+    uint16_t* __restrict__ t, int64_t ldt) {
   const int lane = threadIdx.x & 63;
   const int64_t m = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int nvec = K >> 3;
@@ -109,6 +121,15 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(
     const int idx = c * 64 + lane;
     v[c] = live && idx < nvec ? __builtin_nontemporal_load(xr + idx) : v4u{0u, 0u, 0u, 0u};
   }
+  float pv[PARTS ? kMaxParts / 2 : 1];
+  if constexpr (PARTS) {
+#pragma unroll
+    for (int u = 0; u < kMaxParts / 2; ++u) {   // all in flight at once; a lane past the last one reads it again
+      const int p = 2 * u + (lane >> 5);
+      pv[u] = *reinterpret_cast<const float*>(q + lr_part_offset(m, min(p, parts - 1), lane & 31, K >> 6));
+      if (p >= parts) pv[u] = 0.0f;
+    }
+  }
   us2 mx2 = {0, 0};
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
@@ -122,6 +143,14 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(
   const float a = fmaxf(absmax_from_bits<DT>(mx), 1e-8f);
   const float sc = __fdiv_rn(a, 127.0f);
   const float rc = __fdiv_rn(1.0f, sc);
+  if constexpr (PARTS) {
+    float tv = pv[0];
+#pragma unroll
+    for (int u = 1; u < kMaxParts / 2; ++u) tv += pv[u];
+    tv += __shfl_xor(tv, 32, 64);
+    asm volatile("" : "+v"(tv) : : "memory");   // the partial sums have been read: their bytes may take the codes
+    if (lane < 32) t[m * ldt + lane] = (uint16_t)f32_to_16_bits<DT>(tv);
+  }
   v2u* __restrict__ qr = reinterpret_cast<v2u*>(q + m * (int64_t)K);
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
@@ -180,6 +209,26 @@ __global__ __launch_bounds__(256) void quant_rows_scalar_kernel(
   if (lane == 0) s[m] = sc;
 }
 
+// The quantizer that finishes t from `parts` partial sums (packed codes, K % 64 == 0, aligned rows).
+template <int DT>
+int launch_quant_parts(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t x_rows, const int32_t* row_idx, int8_t* q,
+                       float* s, int32_t* zero9, int parts, void* t, int64_t ldt, hipStream_t stream) {
+  const int64_t rows = (M + 15) & ~15LL;
+  if (const int st = check_grid((rows + 3) / 4, 256, "quant_rows")) return st;
+  const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+  const int need = (int)((K / 8 + 63) / 64);
+#define PQ_QPCASE(C)                                                                                                    \
+  if (need <= C) {                                                                                                     \
+    hipLaunchKernelGGL((quant_rows_vec_kernel<DT, C, true, true>), grid, block, 0, stream,                              \
+                       static_cast<const uint16_t*>(x), ldx, (int)K, M, row_idx, q, s, x_rows, zero9, parts,           \
+                       static_cast<uint16_t*>(t), ldt);                                                                \
+    return check_launch("quant_rows_vec");                                                                             \
+  }
+  PQ_QPCASE(16) PQ_QPCASE(20) PQ_QPCASE(24) PQ_QPCASE(30)
+#undef PQ_QPCASE
+  return set_error(PQ_ESHAPE, "quant_rows: K=%lld too large", (long long)K);
+}
+
 template <int DT, bool PACKED>
 int launch_quant(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t x_rows, const int32_t* row_idx, int8_t* q,
                  float* s, int32_t* zero9, hipStream_t stream) {
@@ -194,7 +243,7 @@ int launch_quant(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t x_row
 #define PQ_QCASE(C)                                                                                       \
   if (need <= C) {                                                                                        \
     hipLaunchKernelGGL((quant_rows_vec_kernel<DT, C, PACKED>), grid, block, 0, stream, xp, ldx, (int)K, M, \
-                       row_idx, q, s, x_rows, zero9);                                                     \
+                       row_idx, q, s, x_rows, zero9, 0, nullptr, 0);                                      \
     return check_launch("quant_rows_vec");                                                                \
   }
     PQ_QCASE(1) PQ_QCASE(2) PQ_QCASE(3) PQ_QCASE(4) PQ_QCASE(5) PQ_QCASE(6) PQ_QCASE(8) PQ_QCASE(10)
@@ -773,23 +822,26 @@ __global__ __launch_bounds__(256) void pack_lowrank_l1t_kernel(const v4u* __rest
 // quant_rows_vec_kernel); then for each 512-wide K slab e:
 //   a. the wave writes its two rows' chunk e into the x slab buffer (16 rows, double buffered);
 //   c. quantizes chunk e and stores its codes (packed K64);
-//   -- barrier (the x slab is complete, and the L1^T slab e, DMA'd one slab ahead, has landed) --
-//   b. issues the LDS-DMA of the L1^T slab e + 1 (32 rows of 1 KB, double buffered);
+//   -- barrier (the x slab is complete, and the L1^T slab e, DMA'd two slabs ahead, has landed) --
+//   b. issues the LDS-DMA of the L1^T slab e + 2 (32 rows of 1 KB, three buffers);
 //   d. reads its 64-wide share of slab e for all 16 rows and the matching L1^T fragments (LDS) and runs
 //      v_mfma_f32_16x16x32 into its t partial.
 // The 8 waves' t partials are summed in LDS in wave order, (..(p0 + p1) ..) + p7, and rounded to 16 bits.
 // Batches are software-pipelined through the registers: after chunk e of batch b is in LDS and quantized, the wave
-// loads chunk e of its next batch into the same registers, so the next rows stream in under this batch's work.
-// Ordering: the L1^T DMA of slab e + 1 is issued after barrier e, when every wave has read that buffer's previous slab
-// (e - 1); it must land before barrier e + 1, and the only vector-memory instructions issued after it are slab e + 1's
-// RPW code stores and RPW next-batch loads, hence vmcnt(2 RPW) there (vector-memory instructions retire in issue
-// order). The slab is straight-line code, so scheduling fences hold the DMA, those stores and loads, and the wait in
-// that order.
-// Past the last batch the next-batch loads read this batch's rows again (discarded), which keeps that count exact.
+// loads chunk e of its next batch into the same registers, so the next rows stream in under this batch's work. The
+// last batch of a workgroup loads nothing.
+// Ordering: the L1^T DMA of slab e + 2 is issued after barrier e, when every wave has read that buffer's previous slab
+// (e - 1); slab e + 2 must land before barrier e + 2. Vector-memory instructions retire in issue order, so the wait
+// there is for all but the instructions issued after that DMA: the RPW code stores and RPW next-batch loads of slabs
+// e + 1 and e + 2 and the DMA of slab e + 3. Two slabs ahead, the wait leaves a slab's loads from memory in flight
+// (one ahead, it waited for them). The slab is straight-line code, so
+// scheduling fences hold the DMA, those stores and loads, and the wait in that order.
 constexpr int kWideWaves = 8;                 // waves per workgroup, two rows each: batches of 16 rows
 constexpr int kWideSlab = 512;                // K elements per slab
 constexpr int kWidePitch = 2 * kWideSlab + 16;   // LDS row pitch: consecutive rows 16 bytes apart in the bank window
 constexpr int kWideRedPitch = 36;             // floats per row of the partial-sum buffer
+constexpr int kWideGrid = 256;                // workgroups, one per CU
+constexpr int64_t kTailRows = 1024;           // rows past whole rounds that take the partial-sum kernel instead
 
 template <int DT, int NCH, int RPW>   // NCH = K / 512: 16-byte chunks per lane per row, and slabs; RPW rows per wave
 __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
@@ -802,9 +854,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
   constexpr int KW = kWideSlab / kWideWaves;   // 64: each wave's share of a slab, two MFMA K steps
   constexpr int BR = kWideWaves * RPW;         // rows per batch (16 or 8)
   static_assert(RPW == 1 || RPW == 2, "rows per wave");
-  // double buffers as separate arrays, so that the compiler can tell an LDS read of one buffer from a pending
+  // the buffers as separate arrays, so that the compiler can tell an LDS read of one buffer from a pending
   // LDS-DMA into the other (it waits for every DMA that may alias a read)
-  __shared__ __attribute__((aligned(1024))) uint8_t lbuf0[32 * kWidePitch], lbuf1[32 * kWidePitch];   // L1^T slabs
+  __shared__ __attribute__((aligned(1024))) uint8_t lbuf0[32 * kWidePitch], lbuf1[32 * kWidePitch], lbuf2[32 * kWidePitch];   // L1^T
   __shared__ __attribute__((aligned(16))) uint8_t xbuf0[16 * kWidePitch], xbuf1[16 * kWidePitch];     // x slabs
   __shared__ __attribute__((aligned(16))) float red[kWideWaves][16][kWideRedPitch];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -820,13 +872,13 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
   }
   const __amdgpu_buffer_rsrc_t rs_l =
       __builtin_amdgcn_make_buffer_rsrc((void*)l1t, (short)0, 32 * K * 2, kBufferWord3);
-  // L1^T slab e -> lbuf[e & 1]: wave w copies rows 4 w .. 4 w + 3, one 1 KB LDS-DMA each; the slab's offset rides
+  // L1^T slab e -> buffer e % 3: wave w copies rows 4 w .. 4 w + 3, one 1 KB LDS-DMA each; the slab's offset rides
   // the scalar offset operand, so the per-lane offsets stay four registers
   const int voff_l = 4 * wave * K * 2 + lane * 16;
   auto dma_l = [&](int e) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_l, (lds_void_t*)((e & 1 ? lbuf1 : lbuf0) + (4 * wave + i) * kWidePitch), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_l, (lds_void_t*)((e % 3 == 0 ? lbuf0 : e % 3 == 1 ? lbuf1 : lbuf2) + (4 * wave + i) * kWidePitch), 16,
                                                voff_l + i * K * 2, e * kWideSlab * 2, 0, 0);
   };
 
@@ -862,20 +914,22 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
     }
   }
   for (int b = blockIdx.x; b < nbatch; b += gridDim.x) {
-    const int bn = b + gridDim.x;   // the next batch (past the end: this batch's rows again, loaded and discarded)
+    const int bn = b + gridDim.x;   // the next batch
+    const bool more = bn < nbatch;
     int64_t mrow[RPW];
     const v4u* xn[RPW];
 #pragma unroll
     for (int rho = 0; rho < RPW; ++rho) {
       mrow[rho] = (int64_t)b * BR + RPW * wave + rho;
-      xn[rho] = src_row(bn < nbatch ? bn : b, rho);
+      xn[rho] = src_row(more ? bn : b, rho);
       if (!live[rho]) {   // a padding row or a gathered row outside x: it quantizes as zeros
 #pragma unroll
         for (int c = 0; c < NCH; ++c) v[rho][c] = v4u{0u, 0u, 0u, 0u};
       }
-      live[rho] = src_of(bn < nbatch ? bn : b, rho) >= 0;   // the batch whose loads xn starts
+      live[rho] = src_of(more ? bn : b, rho) >= 0;   // the batch whose loads xn starts
     }
-    dma_l(0);   // lands before slab 0's barrier: only that slab's code stores and next-batch loads come after it
+    dma_l(0);
+    dma_l(1);
     __builtin_amdgcn_sched_barrier(0);   // (and none of them before it: the vmcnt count below rests on the order)
     float sc[RPW], rc[RPW];
 #pragma unroll
@@ -905,7 +959,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
 #pragma unroll
     for (int e = 0; e < NCH; ++e) {
       uint8_t* const xs = e & 1 ? xbuf1 : xbuf0;
-      const uint8_t* const ls = e & 1 ? lbuf1 : lbuf0;
+      const uint8_t* const ls = e % 3 == 0 ? lbuf0 : e % 3 == 1 ? lbuf1 : lbuf2;
 #pragma unroll
       for (int rho = 0; rho < RPW; ++rho)
         *reinterpret_cast<v4u*>(xs + (RPW * wave + rho) * kWidePitch + lane * 16) = v[rho][e];
@@ -914,16 +968,28 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
 #pragma unroll
       for (int rho = 0; rho < RPW; ++rho)
         *reinterpret_cast<v2u*>(qbatch + rho * 64 + e * 8192 + qlane[rho]) = quant_chunk<DT>(v[rho][e], sc[rho], rc[rho]);
-      // chunk e of the next batch into the registers just freed
+      // chunk e of the next batch into the registers just freed; then this wave's DMA of L1^T slab e has landed: all but
+      // the stores and loads of this slab and the last, and the DMA of slab e + 1
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int kAhead = 4, kStores = RPW;
+      if (more) {
 #pragma unroll
-      for (int rho = 0; rho < RPW; ++rho) v[rho][e] = __builtin_nontemporal_load(xn[rho] + e * 64 + lane);
-      __builtin_amdgcn_sched_barrier(0);   // the slab's stores and loads stay between the DMA and this wait
-      wait_vmcnt<2 * RPW>();   // this wave's DMA of L1^T slab e has landed (RPW stores, RPW loads after it)
+        for (int rho = 0; rho < RPW; ++rho) v[rho][e] = __builtin_nontemporal_load(xn[rho] + e * 64 + lane);
+        __builtin_amdgcn_sched_barrier(0);
+        if (e == 0) wait_vmcnt<2 * kStores + kAhead>();
+        else if (e + 1 < NCH) wait_vmcnt<4 * kStores + kAhead>();
+        else wait_vmcnt<4 * kStores>();
+      } else {
+        if (e == 0) wait_vmcnt<kStores + kAhead>();
+        else if (e + 1 < NCH) wait_vmcnt<2 * kStores + kAhead>();
+        else wait_vmcnt<2 * kStores>();
+      }
+      __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave's x slab writes are done
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_barrier();         // both slabs complete; every wave is done with slab e - 1
       __builtin_amdgcn_sched_barrier(0);
-      if (e + 1 < NCH) dma_l(e + 1);
+      if (e + 2 < NCH) dma_l(e + 2);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ks = 0; ks < KW / 32; ++ks) {
@@ -964,6 +1030,77 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
       if (mo < M) *reinterpret_cast<uint32_t*>(t + mo * ldt + rr) = pack2<DT>(v0, v1);
     }
   }
+}
+
+// ---- rank-32 partial sums for few wide rows --------------------------------------------------------------------------
+// t = x @ L1 (fp32 partial sums of it) spread over the whole chip when there are too few rows to give every CU a
+// batch of quant_lowrank_wide_kernel: workgroup (mb, p) takes rows 32 mb .. + 31 and the p-th of `parts` K ranges, its
+// 4 waves a quarter of the range each, summed in LDS in wave order. The partial sums wait in the packed code buffer
+// (lr_part_offset), whose rows the quantizer that follows reads before it writes their codes: no scratch memory and no
+// synchronisation between workgroups. x is read twice in all (the second time from the caches). Bound by latency: 7.0 us
+// at 512 rows of K = 12288, 16 parts (256 workgroups, 3 K blocks of 8 KB in flight per wave), and the quantizer after
+// it 7.5 us, against 27.0 us for a batch of the wide kernel on 32 CUs.
+// Operands go straight from memory to the MFMA fragments: in each 64-wide K block lane (row l % 32, half l / 32) holds
+// the 32 elements from 32 (l / 32), 16 bytes per MFMA step, of x and of L1^T alike, so a step contracts 16 distinct K
+// and a lane's four steps read 64 contiguous bytes.
+template <int DT>
+__global__ __launch_bounds__(256) void lowrank_partial_kernel(
+    const uint16_t* __restrict__ x, int64_t ldx, int64_t x_rows, int K, int64_t M, const int32_t* __restrict__ row_idx,
+    const uint16_t* __restrict__ l1t, int8_t* __restrict__ qp, int parts) {
+  constexpr int kPitch = 36;   // floats per row of the LDS sums
+  __shared__ __attribute__((aligned(16))) float red[4][32][kPitch];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t mb = blockIdx.x / parts;
+  const int part = (int)(blockIdx.x - mb * parts);
+  const int KT = K >> 6, nr = 4 * parts, ir = 4 * part + wave;   // this wave's K range: blocks [c0, c1)
+  const int c0 = (int)((int64_t)ir * KT / nr), c1 = (int)((int64_t)(ir + 1) * KT / nr);
+  const int64_t m = mb * 32 + (lane & 31);
+  const int64_t src = m >= M ? -1 : row_idx ? (int64_t)row_idx[m] : m;
+  const bool live = src >= 0 && src < x_rows;   // rows past M and gathered rows outside x read as zeros
+  const int kh = (lane >> 5) * 32;
+  const uint16_t* __restrict__ xr = x + (live ? src : 0) * ldx + kh;
+  const uint16_t* __restrict__ lr = l1t + (int64_t)(lane & 31) * K + kh;
+  v16f acc = v16f{};
+  // three K blocks of both operands in flight
+  v4u xb[3][4], lb[3][4];
+  auto load = [&](int j, int c) {
+    if (c >= c1) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      xb[j][e] = *reinterpret_cast<const v4u*>(xr + c * 64 + e * 8);
+      lb[j][e] = *reinterpret_cast<const v4u*>(lr + c * 64 + e * 8);
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < 3; ++j) load(j, c0 + j);
+  for (int c = c0; c < c1; c += 3) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      if (c + j < c1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const v4u xv = live ? xb[j][e] : v4u{0u, 0u, 0u, 0u};
+          if constexpr (DT == PQ_BF16)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, lb[j][e]), __builtin_bit_cast(v8bf, xv), acc, 0, 0, 0);
+          else
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, lb[j][e]), __builtin_bit_cast(v8h, xv), acc, 0, 0, 0);
+        }
+        load(j, c + j + 3);
+      }
+    }
+  }
+  // D[r][row]: the lane holds row l % 32 and r = 8 q + 4 (l / 32) + (0..3)
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    *reinterpret_cast<v4f*>(&red[wave][lane & 31][8 * q + 4 * (lane >> 5)]) =
+        v4f{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  __syncthreads();
+  const int row = tid >> 3, r4 = (tid & 7) * 4;
+  v4f sum = *reinterpret_cast<const v4f*>(&red[0][row][r4]);
+#pragma unroll
+  for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(&red[w][row][r4]);
+  if (mb * 32 + row < M) *reinterpret_cast<v4f*>(qp + lr_part_offset(mb * 32 + row, part, r4, KT)) = sum;
 }
 
 // ---- dequant epilogue over a materialised int32 accumulator ----------------------------------------------
@@ -1131,24 +1268,59 @@ int pq::quant_rows_lowrank_z(const void* x, int32_t x_dtype, int64_t M, int64_t 
                     (uintptr_t)l1t % 16 == 0 && (uintptr_t)t % 4 == 0 && (uintptr_t)qp % 16 == 0 &&
                     (x_dtype == PQ_BF16 || x_dtype == PQ_F16);
   if (wide) {
-    // batches of 16 rows (two per wave) or 8 (one per wave), covering the packed padding rows up to a multiple of 16
-    const int rpw = K <= 12288 ? 2 : 1;
-    const int nbatch = (int)((M + 15) / 16) * (2 / rpw);
-    const dim3 grid((unsigned)std::min(nbatch, 256));
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     const uint16_t* lp = static_cast<const uint16_t*>(l1t);
     uint16_t* tp = static_cast<uint16_t*>(t);
+    // batches of 16 rows (two per wave) or 8 (one per wave), one workgroup per CU
+    const int rpw = K <= 12288 ? 2 : 1;
+    const int64_t round = (int64_t)kWideGrid * kWideWaves * rpw;
+    // Rows past the last whole round. A batch takes its time however few there are (K = 12288: 25-29 us, 24 slabs of
+    // L1^T one after the other), so up to kTailRows of them go to the partial-sum kernel and the quantizer instead,
+    // which spread them over the chip: 14.5 us at 512 rows (27.0), 21.1 at 1024 (28.4), and from there the second read of
+    // x costs more than the short round (2048: 32.3 against 30.0). K = 8192: 11.9 us at 512 rows (18.3), 15.6 at 1024
+    // (19.6); K = 15360: 18.6 (25.0), 23.7 (26.9); at K = 4096 the two kernels gain nothing (9.5 against 10.6 us with a
+    // launch more).
+    const int64_t tail = K >= 8192 && M % round <= kTailRows ? M % round : 0;
+    const int64_t Mw = M - tail;
+    if (Mw > 0) {
+      // covering the packed padding rows up to a multiple of 16
+      const int nbatch = (int)((Mw + 15) / 16) * (2 / rpw);
+      const dim3 grid((unsigned)std::min(nbatch, kWideGrid));
+      int st = PQ_ESHAPE;
 #define PQ_QWCASE(D, NCH, RPW)                                                                                 \
-    if (x_dtype == D && K == 512 * NCH) {                                                                      \
-      hipLaunchKernelGGL((quant_lowrank_wide_kernel<D, NCH, RPW>), grid, dim3(64 * kWideWaves), 0, stream, xp,    \
-                         ldx, x_rows, M, row_idx, lp, qp, s, tp, ldt, nbatch, zero9);                          \
-      return check_launch("quant_rows_lowrank");                                                               \
-    }
-    PQ_QWCASE(PQ_BF16, 8, 2) PQ_QWCASE(PQ_BF16, 12, 2) PQ_QWCASE(PQ_BF16, 16, 2) PQ_QWCASE(PQ_BF16, 20, 2)
-    PQ_QWCASE(PQ_BF16, 24, 2) PQ_QWCASE(PQ_BF16, 30, 1)
-    PQ_QWCASE(PQ_F16, 8, 2) PQ_QWCASE(PQ_F16, 12, 2) PQ_QWCASE(PQ_F16, 16, 2) PQ_QWCASE(PQ_F16, 20, 2)
-    PQ_QWCASE(PQ_F16, 24, 2) PQ_QWCASE(PQ_F16, 30, 1)
+      if (x_dtype == D && K == 512 * NCH) {                                                                    \
+        hipLaunchKernelGGL((quant_lowrank_wide_kernel<D, NCH, RPW>), grid, dim3(64 * kWideWaves), 0, stream, xp,  \
+                           ldx, x_rows, Mw, row_idx, lp, qp, s, tp, ldt, nbatch, zero9);                       \
+        st = check_launch("quant_rows_lowrank");                                                               \
+      }
+      PQ_QWCASE(PQ_BF16, 8, 2) PQ_QWCASE(PQ_BF16, 12, 2) PQ_QWCASE(PQ_BF16, 16, 2) PQ_QWCASE(PQ_BF16, 20, 2)
+      PQ_QWCASE(PQ_BF16, 24, 2) PQ_QWCASE(PQ_BF16, 30, 1)
+      PQ_QWCASE(PQ_F16, 8, 2) PQ_QWCASE(PQ_F16, 12, 2) PQ_QWCASE(PQ_F16, 16, 2) PQ_QWCASE(PQ_F16, 20, 2)
+      PQ_QWCASE(PQ_F16, 24, 2) PQ_QWCASE(PQ_F16, 30, 1)
 #undef PQ_QWCASE
+      if (st != PQ_OK || tail == 0) return st;
+      zero9 = nullptr;   // (written by the launch above)
+    }
+    // the tail's rows: Mw is a multiple of 16, so they start a row block of the packed codes
+    const uint16_t* const xt = row_idx ? xp : xp + Mw * ldx;
+    const int64_t xt_rows = row_idx ? x_rows : x_rows - Mw;
+    const int32_t* const rt = row_idx ? row_idx + Mw : nullptr;
+    int8_t* const qt = qp + Mw * K;
+    // K ranges per row: 16, or 8 where 16 would be more workgroups than the chip runs at once with the fewer (1024
+    // rows: 21.1 against 21.9 us at K = 12288)
+    const int parts = tail <= 768 ? kMaxParts : kMaxParts / 2;
+    const dim3 grid((unsigned)((tail + 31) / 32 * parts)), block(256);
+    if (x_dtype == PQ_BF16)
+      hipLaunchKernelGGL(lowrank_partial_kernel<PQ_BF16>, grid, block, 0, stream, xt, ldx, xt_rows, (int)K, tail, rt, lp,
+                         qt, parts);
+    else
+      hipLaunchKernelGGL(lowrank_partial_kernel<PQ_F16>, grid, block, 0, stream, xt, ldx, xt_rows, (int)K, tail, rt, lp,
+                         qt, parts);
+    if (const int st = check_launch("lowrank_partial")) return st;
+    if (x_dtype == PQ_BF16)
+      return launch_quant_parts<PQ_BF16>(xt, tail, K, ldx, xt_rows, rt, qt, s + Mw, zero9, parts, tp + Mw * ldt, ldt,
+                                         stream);
+    return launch_quant_parts<PQ_F16>(xt, tail, K, ldx, xt_rows, rt, qt, s + Mw, zero9, parts, tp + Mw * ldt, ldt, stream);
   }
   if (!fused) {
     const int st = pq::quant_rows_packed_z(x, x_dtype, M, K, ldx, x_rows, row_idx, qp, s, zero9, stream);

@@ -232,3 +232,42 @@ def test_int8linear_fragment_order_follows_lr_At(cuda):
     y_plain = q1(x)
     assert torch.equal(y_frag.view(torch.int16), y_plain.view(torch.int16))
     assert not torch.equal(y_frag.view(torch.int16), y2.view(torch.int16))
+
+
+@pytest.mark.parametrize("gather", [False, True])
+@pytest.mark.parametrize("M,K,dtype", [
+    # the whole call through the partial sums: one row, around 16- and 32-row blocks, both part counts, the last size
+    (1, 12288, torch.bfloat16), (33, 8192, torch.float16), (512, 12288, torch.bfloat16), (768, 15360, torch.bfloat16),
+    (769, 10240, torch.bfloat16), (1024, 12288, torch.float16), (1025, 12288, torch.bfloat16),
+    # whole rounds (4096 rows; 2048 at K = 15360) and a tail
+    (4097, 8192, torch.bfloat16), (4096 + 1000, 12288, torch.bfloat16), (4096 + 1025, 8192, torch.float16),
+    (2048 + 17, 15360, torch.bfloat16), (8192, 8192, torch.bfloat16)])
+def test_quant_rows_lowrank_wide_tail(cuda, gather, M, K, dtype):
+    """The wide-row rule: rows past the last whole round of one batch per CU take lowrank_partial_kernel and the
+    quantizer that finishes t. Codes and scales as the plain quantizer's, bit for bit; t within one 16-bit rounding of
+    the float64 product (2^-8 |t| in bf16) plus the fp32 sum's error (K 2^-24 sum |x l1|); gathered rows outside x
+    read as zeros; nothing beside t's own columns is written."""
+    from pyraquant_amd import int8_exec as E
+    from pyraquant_amd.workloads import make_x
+
+    rows = M + 5
+    x = make_x(rows, K, dtype, seed=M + K, device=cuda)
+    l1t = _l1(K, 32, dtype, K).t().contiguous().to(cuda)
+    idx = None
+    if gather:
+        g = torch.Generator().manual_seed(M)
+        idx = torch.randint(0, rows, (M,), generator=g, dtype=torch.int32)
+        idx[0], idx[M // 2] = rows, -1
+        idx = idx.to(cuda)
+    xin = x if gather else x[:M]
+    qp, s, t = E.quant_rows_lowrank(xin, l1t, idx)
+    qr, sr = E.quant_rows_packed(xin, idx)
+    assert torch.equal(qp, qr) and torch.equal(s, sr)
+    xs = x[:M] if idx is None else torch.where(((idx >= 0) & (idx < rows))[:, None], x[idx.clamp(0, rows - 1).long()],
+                                               torch.zeros((), dtype=dtype, device=cuda))
+    for r0 in range(0, M, 2048):
+        xd = xs[r0:r0 + 2048].double()
+        ref = xd @ l1t.double().t()
+        bound = ref.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + \
+            K * 2.0 ** -24 * (xd.abs() @ l1t.double().abs().t()) + 1e-7
+        assert bool(((t[r0:r0 + 2048].double() - ref).abs() <= bound).all())
