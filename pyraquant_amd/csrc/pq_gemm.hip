@@ -940,6 +940,112 @@ void gemm_dma_kernel(const GemmArgs p) {
   }
 }
 
+// ---- few blocks: K split over the waves of a workgroup ---------------------------------------------------------
+// For outputs of few blocks (packed operands, per-channel scales). In gemm_dma_kernel's 128 x 64 blocks such a product
+// ran on a fraction of the CUs, one wave per SIMD and K stage after K stage behind a barrier: 154 x 2048 x 1280 took
+// 8.7 us in 30 blocks, bound by the latency of 32 stages in a row. Here every wave of a (32 TI) x (32 TJ) block (n x m)
+// holds the whole block's accumulators for the stages w, w + NW, .. of K, loads its fragments straight from memory into
+// registers, D stages ahead, and meets no barrier until the end, where the NW partial sums are added in LDS (whole
+// numbers: the order does not matter) and the epilogue's units (ET weight tiles x 32 rows) are dealt to the waves.
+// 5.5 us at that size (100 blocks, 8 stages a wave).
+// Fragments: lane l reads row l % 32 of a 32-row fragment, K chunk 2 s + l / 32 of substep s: in the packed layout the
+// two 1 KB blocks of the fragment's rows, 16 bytes a lane. Row blocks past the operand's last are read as the last one
+// (their outputs are not stored), and stages past K as the last stage (their products are not taken), so every load is
+// in bounds and none is conditional.
+template <int TI, int TJ, int NW, int D, int LRS, int DT, bool ACC>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW), amdgpu_waves_per_eu(NW / 2, NW / 2)))
+void gemm_ksplit_kernel(const GemmArgs p) {
+  constexpr int BN = 32 * TI, BM = 32 * TJ, NF = TI + TJ;
+  constexpr int ET = TI % 2 == 0 && (TI / 2) * TJ >= NW ? 2 : 1;
+  constexpr int NU = TI / ET * TJ;                  // epilogue units, unit u on wave u % NW
+  using Epi = Epilogue<ET, 1, kModeChannel, LRS, DT, DT, 1, false, ACC>;
+  constexpr int TILE = 4096;                        // bytes of a tile's int32 accumulators
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[NW * TI * TJ * TILE];
+  static_assert(Epi::kStageBytes <= ET * TILE, "a unit's output staging fits its own tiles' partial sums");
+  static_assert(2 * sizeof(smem) <= 160 * 1024, "two workgroups per CU");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tm, tn;
+  tile_coords<8>(blockIdx.x, p.tiles_m * p.tiles_n, p.tiles_m, p.tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int KT = p.K / kBKd;
+  const int nb_w = (min(BN, p.N - n0) + 15) / 16, nb_a = (min(BM, p.M - m0) + 15) / 16;   // 16-row blocks
+  const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.w + (int64_t)(n0 / 16) * KT * 1024), (short)0, nb_w * KT * 1024, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.a + (int64_t)(m0 / 16) * KT * 1024), (short)0, nb_a * KT * 1024, kBufferWord3);
+  // byte offset of this lane's chunk of substep 0 in stage 0 of each fragment (substep 1: bit 5 flipped)
+  const int r16 = lane & 15, half = (lane >> 4) & 1;
+  const int lo = r16 * 64 + (((lane >> 5) ^ k64_swz(r16)) << 4);
+  int vo[NF];
+#pragma unroll
+  for (int i = 0; i < TI; ++i) vo[i] = min(2 * i + half, nb_w - 1) * KT * 1024 + lo;
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) vo[TI + j] = min(2 * j + half, nb_a - 1) * KT * 1024 + lo;
+  v4i f[D][2][NF];
+  auto load = [&](int d, int kt) {
+    const int so = min(kt, KT - 1) * 1024;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < NF; ++i)
+        f[d][s][i] = __builtin_bit_cast(
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(i < TI ? rs_w : rs_a, vo[i] ^ (s * 32), so, 0));
+  };
+  v16i acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = v16i{};
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, wave + NW * d);
+  for (int kt = wave; kt < KT;) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (kt < KT) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[d][s][i], f[d][s][TI + j], acc[i][j], 0, 0, 0);
+      }
+      load(d, kt + NW * D);
+      kt += NW;
+    }
+  }
+  // partial sums: 16 bytes per lane and quarter of a tile, a unit's tiles side by side
+  v4i* const red = reinterpret_cast<v4i*>(smem);
+#pragma unroll
+  for (int j = 0; j < TJ; ++j)
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        red[((wave * TJ + j) * TI + i) * 256 + q * 64 + lane] =
+            v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  __syncthreads();
+  for (int u = wave; u < NU; u += NW) {
+    const int j = u / (TI / ET), i0 = u % (TI / ET) * ET;
+    Epi epi;
+    epi.prefetch_rows(p, m0 + 32 * j, lane);
+    v16i y[ET][1];
+#pragma unroll
+    for (int i = 0; i < ET; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v4i v = red[(j * TI + i0 + i) * 256 + q * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += red[((w * TJ + j) * TI + i0 + i) * 256 + q * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[i][0][4 * q + e] = v[e];
+      }
+    // the staging takes the place of wave 0's partial sums of this unit, which no other wave reads
+    epi.run(p, y, n0 + 32 * i0, m0 + 32 * j, lane, smem + (j * TI + i0) * TILE);
+  }
+}
+
 // ---- launchers ---------------------------------------------------------------------------------------------
 int grid_of(GemmArgs& a, int BM, int BN, int threads, dim3& grid) {
   a.tiles_m = (a.M + BM - 1) / BM;
@@ -1003,6 +1109,14 @@ int launch_dma(GemmArgs& a, hipStream_t stream) {
   return check_launch("int8_gemm");
 }
 
+template <int TI, int TJ, int NW, int D, int LRS, int DT, bool ACC>
+int launch_ksplit(GemmArgs& a, hipStream_t stream) {
+  dim3 grid;
+  if (const int st = grid_of(a, 32 * TJ, 32 * TI, 64 * NW, grid)) return st;
+  hipLaunchKernelGGL((gemm_ksplit_kernel<TI, TJ, NW, D, LRS, DT, ACC>), grid, dim3(64 * NW), 0, stream, a);
+  return check_launch("int8_gemm");
+}
+
 // 128 x 128 blocks of the problem (the small-problem tile).
 inline int64_t small_blocks(const GemmArgs& a) { return (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128); }
 
@@ -1041,6 +1155,16 @@ int dispatch_tiles(GemmArgs& a, hipStream_t stream) {
       return launch_dma<2, 2, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     }
   } else {
+    // so few outputs that 64 x 32 or 64 x 64 blocks fit the CUs at once: K split over each block's waves
+    // (gemm_ksplit_kernel). The old blocks at the same sizes, M x K x N: 154 x 2048 x 1280 8.7 us, 5.5 now (64 x 32
+    // blocks; 6.0 in 64 x 64), 512 x 640 x 640 5.6 and 4.6, 128 x 3072 x 3072 11.2 and 7.3; 256 x 3072 x 3072 11.6, now
+    // 9.3 (64 x 64; 11.2 in 384 blocks of 64 x 32), 512 x 5120 x 1280 15.6 and 13.0, 256 x 12288 x 3072 31.4 and 22.9. Past
+    // one block per CU the larger blocks win: 1024 x 1280 x 1280 7.7 against 10.0 us, 128 x 3072 x 9216 12.1 against 15.1.
+    if constexpr (PACKED && MODE == kModeChannel) {
+      const int64_t cus = persistent_workgroups(stream), bn = (a.N + 63) / 64;
+      if ((a.M + 31) / 32 * bn <= cus) return launch_ksplit<2, 1, 4, 4, LRS, ODT, ACC>(a, stream);
+      if ((a.M + 63) / 64 * bn <= cus) return launch_ksplit<2, 2, 4, 4, LRS, ODT, ACC>(a, stream);
+    }
     if (big_tiles(a, stream)) return launch_dma<4, 2, 4, 1, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     // fewer 128 x 128 blocks than half the CUs: 128 x 64 blocks (measured 1.3x faster at 80 blocks, even at 160)
     if (small_blocks(a) < 128) return launch_dma<2, 1, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);

@@ -350,3 +350,36 @@ def test_gemm_deep_k_tiles(oracle, cuda, packed):
     yp = E.int8_gemm_packed(E.pack_k64(a), s_row, E.pack_k64(w), s_w, bias, M, N, K, torch.bfloat16, t=t, l2t=l2t)
     yr = E._gemm(a, s_row, w, s_w, 0, bias, t, l2t, torch.bfloat16)
     assert torch.equal(yp, yr)
+
+
+@pytest.mark.parametrize("M,K,N", [
+    # K of 1, 2, 3, 4, 5 and 17 stages over the 4 waves (4 stages ahead); rows and columns around the 64 x 32 and
+    # 64 x 64 blocks; a last n block half filled; the last sizes of either block (256 CUs) and one block more
+    (1, 64, 64), (31, 128, 64), (32, 192, 128), (33, 256, 192), (64, 320, 64), (65, 1088, 704), (154, 2048, 1280),
+    (512, 640, 1024), (513, 640, 1024), (1024, 640, 1024), (1025, 640, 1024), (200, 4096, 2048)])
+@pytest.mark.parametrize("R,dtype,scatter,accumulate", [(0, torch.bfloat16, False, False), (16, torch.float16, True, False),
+                                                        (32, torch.bfloat16, True, True), (64, torch.bfloat16, False, True)])
+def test_few_blocks_split_k(cuda, M, K, N, R, dtype, scatter, accumulate):
+    """Products of few blocks (gemm_ksplit_kernel: K split over a block's waves) against the row-major GEMM, whose
+    blocks and K order are others: whole-number sums and the same epilogue, so equal bit for bit, low rank, bias,
+    scatter and accumulate included; rows that no index names stay as they were."""
+    from pyraquant_amd import int8_exec as E
+
+    g = torch.Generator().manual_seed(M * 7 + K + N + R)
+    a = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).to(cuda)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).to(cuda)
+    sr = (torch.rand(M, generator=g) * 0.05 + 1e-3).to(cuda)
+    sw = (torch.rand(N, generator=g) * 2e-4 + 1e-5).to(cuda)
+    bias = (torch.randn(N, generator=g) * 0.01).to(cuda)
+    t = (torch.randn(M, R, generator=g) * 0.5).to(dtype).to(cuda) if R else None
+    l2t = (torch.randn(N, R, generator=g) * 0.02).to(dtype).to(cuda) if R else None
+    y = E._gemm(a, sr, w, sw, 0, bias, t, l2t, dtype)
+    rows = M + 9
+    idx = torch.randperm(rows, generator=g)[:M].to(torch.int32).to(cuda) if scatter else None
+    canvas = torch.randn(rows if scatter else M, N, generator=g).to(dtype).to(cuda)
+    where = idx.long() if scatter else torch.arange(M, device=cuda)
+    ref = canvas.clone()
+    ref[where] = canvas[where] + y if accumulate else y
+    E.int8_gemm_packed(E.pack_k64(a), sr, E.pack_k64(w), sw, bias, M, N, K, dtype, t=t, l2t=l2t, out=canvas,
+                       out_row_idx=idx, accumulate=accumulate)
+    assert torch.equal(canvas.view(torch.int16), ref.view(torch.int16))
