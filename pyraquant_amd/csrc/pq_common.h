@@ -30,6 +30,11 @@ int quant_rows_lowrank_z(const void* x, int32_t x_dtype, int64_t M, int64_t K, i
                          const int32_t* row_idx, const void* l1t, const void* l1f, int64_t R, int8_t* qp, float* s,
                          void* t, int64_t ldt, int32_t* zero9, hipStream_t stream);
 
+// The whole layer as one kernel where it has few rows (pq_quant.hip): per-channel weights, no low-rank branch. `taken`
+// says whether it was launched.
+int linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,
+                 const float* s_w, const float* bias, void* y, int64_t ldy, int64_t N, bool& taken, hipStream_t stream);
+
 // ---- vector types of the MFMA operands -----------------------------------------------------------------
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));

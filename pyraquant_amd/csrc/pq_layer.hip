@@ -39,6 +39,11 @@ LayerSlices layer_slices(int64_t M, int64_t K, int64_t R) {
 static int run_layer(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,
                      const float* s_w, int64_t group, const float* bias, const void* l1t, const void* l1f, int64_t R,
                      const void* l2t, int64_t Re, void* y, int64_t ldy, int64_t N, uint8_t* ws, hipStream_t stream) {
+  if (R == 0 && group == 0) {
+    bool taken = false;
+    const int st = linear_small(x, x_dtype, M, K, ldx, w_packed, s_w, bias, y, ldy, N, taken, stream);
+    if (taken) return st;
+  }
   const LayerSlices sl = layer_slices(M, K, R);
   int8_t* const q = reinterpret_cast<int8_t*>(ws);
   float* const s = reinterpret_cast<float*>(ws + sl.scales);

@@ -1103,6 +1103,115 @@ __global__ __launch_bounds__(256) void lowrank_partial_kernel(
   if (mb * 32 + row < M) *reinterpret_cast<v4f*>(qp + lr_part_offset(mb * 32 + row, part, r4, KT)) = sum;
 }
 
+// ---- a whole layer of few rows in one kernel --------------------------------------------------------------------------
+// y = Linear(x) for per-channel weights without a low-rank branch, where quantizer and GEMM as two kernels spend their
+// time starting up: at 154 x 2048 x 1280, 3.7 us and 5.9 us (7.5 us here), and a launch more for the host. A workgroup of 8 waves owns 16
+// rows and 64 outputs, quantizes its rows into LDS (two rows per wave, the steps of quant_rows_vec_kernel; the blocks
+// along n repeat that work, which at this size is cheaper than a launch) and multiplies them by its 64 weight rows, K
+// split over the waves: wave w takes the stages w, w + 8, .. of 64, the first kSmallAhead of them loaded before the
+// quantizer starts. v_mfma_i32_16x16x64_i8: a fragment of either operand is one 1 KB block of the packed layout, lane l
+// reading chunk l / 16 of row l % 16, from memory for the weights and from LDS, where the codes lie in the same layout.
+// The 8 partial sums are added in LDS (whole numbers), then dequantized as the GEMM's epilogue does:
+// acc * (s_row * s_w) + bias, rounded to 16 bits.
+constexpr int kSmallRows = 16, kSmallCols = 64, kSmallWaves = 8, kSmallAhead = 4;
+constexpr int kSmallMaxK = 4096;   // 64 KB of codes
+// Most workgroups (16 x 64 outputs each) that still win, against quantizer + GEMM and about 1 us between the two:
+// 154 x 2048 x 1280 (200 workgroups) 7.5 us against 3.7 + 5.9, 77 x 4096 x 1280 (100) 10.1 against 4.4 + 7.6, 512 x 640 x
+// 640 (320) 7.9 against 3.2 + 4.9, 256 x 1280 x 1280 (320) 8.9 against 3.7 + 5.8; then the repeated quantizer work loses:
+// 640 x 2048 x 640 (400) 11.4 against 4.3 + 6.3, 512 x 1280 x 1280 (640) 13.5 against 3.8 + 7.2.
+constexpr int64_t kSmallBlocks = 320;
+
+template <int DT, int CH>   // rows of at most 512 CH elements
+__global__ __launch_bounds__(64 * kSmallWaves) void linear_small_kernel(
+    const uint16_t* __restrict__ x, int64_t ldx, int K, int64_t M, const int8_t* __restrict__ wp,
+    const float* __restrict__ s_w, const float* __restrict__ bias, uint16_t* __restrict__ y, int64_t ldy, int tiles_n) {
+  constexpr int NT = kSmallCols / 16;
+  __shared__ __attribute__((aligned(1024))) uint8_t codes[512 * CH * kSmallRows];
+  __shared__ __attribute__((aligned(16))) v4i red[kSmallWaves][NT][64];
+  __shared__ float srow[kSmallRows];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t tm = blockIdx.x / tiles_n;
+  const int tn = (int)(blockIdx.x - tm * tiles_n);
+  const int KT = K >> 6, nvec = K >> 3;
+  const int r16 = lane & 15;
+  const int lo = r16 * 64 + (((lane >> 4) ^ k64_swz(r16)) << 4);   // this lane's chunk of a fragment's block
+  const int8_t* const wt = wp + (int64_t)tn * NT * KT * 1024 + lo;
+  v4i wf[kSmallAhead][NT];
+  auto load = [&](int d, int kt) {   // (past the end: the last stage again, not used)
+    const int k = min(kt, KT - 1);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) wf[d][i] = *reinterpret_cast<const v4i*>(wt + ((int64_t)i * KT + k) * 1024);
+  };
+  v4u v[2][CH];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t m = tm * kSmallRows + 2 * wave + h;
+    const v4u* xr = reinterpret_cast<const v4u*>(x + min(m, M - 1) * ldx);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int idx = c * 64 + lane;
+      v[h][c] = m < M && idx < nvec ? xr[idx] : v4u{0u, 0u, 0u, 0u};
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < kSmallAhead; ++d) load(d, wave + kSmallWaves * d);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    us2 mx2 = {0, 0};
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mx2 = __builtin_elementwise_max(mx2, __builtin_bit_cast(us2, v[h][c][e] & 0x7fff7fffu));
+    const uint32_t mx = wave_max_u32(mx2.x > mx2.y ? mx2.x : mx2.y);
+    const float sc = __fdiv_rn(fmaxf(absmax_from_bits<DT>(mx), 1e-8f), 127.0f);
+    const float rc = __fdiv_rn(1.0f, sc);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int idx = c * 64 + lane;
+      if (idx < nvec) *reinterpret_cast<v2u*>(codes + k64_offset(2 * wave + h, idx * 8, KT)) = quant_chunk<DT>(v[h][c], sc, rc);
+    }
+    if (lane == 0) srow[2 * wave + h] = sc;
+  }
+  __syncthreads();
+  v4i acc[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) acc[i] = v4i{};
+  for (int kt = wave; kt < KT;) {
+#pragma unroll
+    for (int d = 0; d < kSmallAhead; ++d) {
+      if (kt < KT) {
+        const v4i af = *reinterpret_cast<const v4i*>(codes + kt * 1024 + lo);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[d][i], af, acc[i], 0, 0, 0);
+      }
+      load(d, kt + kSmallWaves * kSmallAhead);
+      kt += kSmallWaves;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NT; ++i) red[wave][i][lane] = acc[i];
+  __syncthreads();
+  if (wave >= NT) return;
+  // wave i finishes weight tile i: D[n][m], the lane holds row m = l % 16 and n = 4 (l / 16) + (0..3)
+  v4i a = red[0][wave][lane];
+#pragma unroll
+  for (int w = 1; w < kSmallWaves; ++w) a += red[w][wave][lane];
+  const int64_t m = tm * kSmallRows + r16;
+  const int n = tn * kSmallCols + wave * 16 + 4 * (lane >> 4);
+  const v4f sw = *reinterpret_cast<const v4f*>(s_w + n);
+  const float sr = srow[r16];
+  float o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (float)a[e] * (sr * sw[e]);
+  if (bias) {
+    const v4f b = *reinterpret_cast<const v4f*>(bias + n);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = o[e] + b[e];
+  }
+  if (m < M) *reinterpret_cast<v2u*>(y + m * ldy + n) = v2u{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
+}
+
 // ---- dequant epilogue over a materialised int32 accumulator ----------------------------------------------
 template <int DT>
 __global__ __launch_bounds__(256) void dequant_epilogue_kernel(
@@ -1346,6 +1455,31 @@ int pq::quant_rows_lowrank_z(const void* x, int32_t x_dtype, int64_t M, int64_t 
   PQ_QLCASE(PQ_F16, 12, 16)
 #undef PQ_QLCASE
   return set_error(PQ_ESHAPE, "pq_quant_rows_lowrank: unsupported shape");
+}
+
+// The layer as one kernel, or `taken` false where its shape, size or alignment is the two kernels'.
+int pq::linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,
+                     const float* s_w, const float* bias, void* y, int64_t ldy, int64_t N, bool& taken,
+                     hipStream_t stream) {
+  const int64_t blocks = (M + kSmallRows - 1) / kSmallRows * (N / kSmallCols);
+  taken = blocks <= kSmallBlocks && K <= kSmallMaxK && K % 64 == 0 && N % kSmallCols == 0 && ldx >= K && ldx % 8 == 0 && ldy >= N &&
+          ldy % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_packed % 16 == 0 && (uintptr_t)s_w % 16 == 0 &&
+          (uintptr_t)bias % 16 == 0 && (uintptr_t)y % 8 == 0 && x && w_packed && s_w && y &&
+          (x_dtype == PQ_BF16 || x_dtype == PQ_F16);
+  if (!taken) return PQ_OK;
+  const dim3 grid((unsigned)blocks), block(64 * kSmallWaves);
+  const uint16_t* xp = static_cast<const uint16_t*>(x);
+  uint16_t* yp = static_cast<uint16_t*>(y);
+#define PQ_SMALL(D, C)                                                                                                  \
+  if (x_dtype == D && K <= 512 * C) {                                                                                  \
+    hipLaunchKernelGGL((linear_small_kernel<D, C>), grid, block, 0, stream, xp, ldx, (int)K, M, w_packed, s_w, bias,   \
+                       yp, ldy, (int)(N / kSmallCols));                                                                \
+    return check_launch("int8_linear");                                                                                \
+  }
+  PQ_SMALL(PQ_BF16, 2) PQ_SMALL(PQ_BF16, 4) PQ_SMALL(PQ_BF16, 8)
+  PQ_SMALL(PQ_F16, 2) PQ_SMALL(PQ_F16, 4) PQ_SMALL(PQ_F16, 8)
+#undef PQ_SMALL
+  return PQ_OK;
 }
 
 extern "C" int pq_pack_lowrank_l1t(const void* l1t, int32_t dtype, int64_t R, int64_t K, void* l1f, hipStream_t stream) {

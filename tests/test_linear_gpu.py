@@ -505,3 +505,32 @@ def test_int8linear_under_inference_mode(cuda):
         y2 = model(x)
     assert torch.equal(y, ref)
     assert torch.equal(y2, ref)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 64, 64), (15, 448, 64), (16, 512, 128), (17, 576, 320), (33, 1024, 640),
+                                   (77, 1088, 1280), (154, 2048, 1280), (31, 2112, 64), (50, 4096, 192),
+                                   (20, 4160, 64), (512, 640, 640), (513, 640, 640)])
+@pytest.mark.parametrize("dtype,bias,pad", [(torch.bfloat16, True, 0), (torch.float16, False, 24)])
+def test_int8linear_few_rows_one_kernel(cuda, M, K, N, dtype, bias, pad):
+    """Layers of few rows run as one kernel (linear_small_kernel): rows and K stages around its 16-row blocks, 8 waves
+    and register sizes, its last K (4096) and last workgroup count (320), padded row strides, an all-zero row, both
+    types; bit-identical to the quantizer and the GEMM as two kernels, and to the codes' product."""
+    from pyraquant_amd import int8_exec as E
+    from pyraquant_amd.workloads import make_linear, make_x
+
+    lin = E.Int8Linear(make_linear(K, N, 0, bias), device=cuda)
+    wide = torch.zeros(M, K + pad, dtype=dtype, device=cuda)
+    wide[:, :K] = make_x(M, K, dtype, seed=M + K).to(cuda)
+    wide[M // 2] = 0
+    x = wide[:, :K]
+    y = lin(x)
+    xq, sx = E.quant_rows_packed(x)
+    ref = E.int8_gemm_packed(xq, sx, lin.weight_packed, lin.w_scale, lin.bias, M, N, K, dtype)
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+    if N <= 320:
+        q, s = E.quant_rows(x)
+        exact = (q.double() @ lin.weight_int8.double().t()) * (s[:, None] * lin.w_scale[None, :]).double()
+        if bias:
+            exact = exact + lin.bias.double()
+        lim = exact.abs() * 2.0 ** (-8 if dtype == torch.bfloat16 else -10) + 1e-6
+        assert bool(((y.double() - exact).abs() <= lim).all())
