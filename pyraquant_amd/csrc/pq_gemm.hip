@@ -67,6 +67,7 @@ struct GemmArgs {
   int M, N, K, R;
   int tiles_m, tiles_n;
   int* sched;         // persistent blocks: 9 ints of claim counters, zero at launch and left zero (or NULL)
+  int whole_lo, whole_hi;   // persistent blocks: tiles that go out whole, of an XCD list of tiles / 8 and of one more
 };
 
 enum { kModeI32 = 0, kModeChannel = 1, kModeGroup32 = 2 };
@@ -496,11 +497,12 @@ constexpr bool persistent_block() {
   return OCC == 1 && TI == 4 && WMW == 4 && !ACC && epilogue_in_ring<TI, TJ, WMW, NS, OCC, MODE, LRS, LRDT, ODT, ACC>();
 }
 
-// WMW waves along m (2 or 4) times 2 along n; OCC workgroups per CU.
-template <int TI, int TJ, int WMW, int NS, int OCC, bool PACKED, int MODE, int LRS, int LRDT, int ODT, bool ACC = false>
-__global__ __attribute__((amdgpu_flat_work_group_size(128 * WMW, 128 * WMW),
-                          amdgpu_waves_per_eu(OCC * WMW / 2, OCC * WMW / 2)))
-void gemm_dma_kernel(const GemmArgs p) {
+// One tile: the output block whose first row and column are m0 and n0, on the whole workgroup. WMW waves along m (2 or
+// 4) times 2 along n; OCC workgroups per CU. `rev` sweeps K backwards; before_epilogue runs between the K loop and the
+// epilogue. smem: NS * STAGE + SLOTS * SB bytes of LDS, which every wave must be done with on entry.
+template <int TI, int TJ, int WMW, int NS, int OCC, bool PACKED, int MODE, int LRS, int LRDT, int ODT, bool ACC, typename F>
+__device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int lane, int wave, int m0, int n0, bool rev,
+                                          F before_epilogue) {
   constexpr bool G32 = MODE == kModeGroup32;
   constexpr int NW = 2 * WMW;                 // waves per workgroup
   constexpr int BN = 64 * TI, BM = 32 * TJ * WMW;
@@ -524,66 +526,14 @@ void gemm_dma_kernel(const GemmArgs p) {
   constexpr int kRest = TI * TJ - NF;         // MFMAs of a substep beyond the NF that carry a fragment read
   constexpr int kVPer = kRest > 0 ? (DPW + kRest - 1) / (kRest > 0 ? kRest : 1) : 0;   // DMA per such MFMA
   static_assert(NS >= 3 && (NS * STAGE + SLOTS * SB) * OCC <= 160 * 1024, "LDS ring");
+  // Ping-pong main loop for the 8-wave blocks (see below); the 4-wave blocks interleave instead.
+  constexpr bool PP = NW == 8 && OCC == 1 && !G32;
   // LDS: the group-32 scale slots first, then the operand ring. With the scales at the start their LDS reads fit the
   // 16-bit immediate offset of ds_read (past a 64 KB ring they cost a v_add each); SLOTS * SB is a multiple of 1 KB.
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[NS * STAGE + SLOTS * SB];
   uint8_t* const sscale = smem;
   uint8_t* const ring = smem + SLOTS * SB;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = wave & 1;
   const int wm = wave >> 1;
-
-  // Persistent blocks (the 256 x 256 tile with its epilogue operands in the ring, no accumulate): one workgroup per
-  // CU loops over tiles, which takes the relaunch gap out of every tile after the first. Virtual block vb is the id
-  // the launch-per-tile grid would have given the tile (tile_coords: XCD vb % 8, its local index vb / 8), so a
-  // workgroup stays on its XCD's tiles and the raster is unchanged. The first tile of workgroup b is vb = b. After
-  // that, with a scheduling buffer (p.sched: 8 per-XCD claim counters and an exit count, zero at launch), a
-  // workgroup claims the next local index of its own XCD's tiles, and once those are gone it claims from the other
-  // XCDs' lists. The XCDs of one chip run the loop at different speeds (up to 5 % apart), so fixed shares finish
-  // up to 165 us apart at c1. Without the buffer it steps vb by the grid size (a fixed share per workgroup).
-  constexpr bool PERSIST = persistent_block<TI, TJ, WMW, NS, OCC, MODE, LRS, LRDT, ODT, ACC>();
-  // Ping-pong main loop for the 8-wave 256 x 256 blocks (see below); the 4-wave blocks interleave instead.
-  constexpr bool PP = NW == 8 && OCC == 1 && !G32;
-  const int nbt = p.tiles_m * p.tiles_n;
-  // Claims (lane 0 of wave 0). XCD x's list holds cnt(x) tiles, of which first(x) went out as first tiles.
-  const int x0 = blockIdx.x & 7;
-  auto xcd_cnt = [&](int x) { return (nbt >> 3) + (x < (nbt & 7) ? 1 : 0); };
-  auto xcd_first = [&](int x) { return ((int)gridDim.x - x + 7) >> 3; };
-  // Part 1, issued before the epilogue so that the atomic's round trip overlaps it: the next local index of the own
-  // XCD's list (or cnt(x0) if the first tiles took them all).
-  auto claim_own = [&]() -> int {
-    if (xcd_first(x0) >= xcd_cnt(x0)) return xcd_cnt(x0);
-    return atomicAdd(p.sched + x0, 1) + xcd_first(x0);
-  };
-  // Part 2, after the epilogue: the own index if the list still had one, else the other 7 lists in a rotated order,
-  // so that stealers spread over the victims. Without a scheduling buffer, the fixed share: vb + grid.
-  auto claim_rest = [&](int vb, int own) -> int {
-    if (!p.sched) return vb + (int)gridDim.x;
-    if (own < xcd_cnt(x0)) return (own << 3) | x0;
-    const int rot = blockIdx.x >> 3;
-    for (int k = 1; k < 8; ++k) {
-      const int x = (x0 + 1 + (k - 1 + rot) % 7) & 7;
-      const int cnt = xcd_cnt(x), first = xcd_first(x);
-      if (first >= cnt) continue;
-      const int li = atomicAdd(p.sched + x, 1) + first;
-      if (li < cnt) return (li << 3) | x;
-    }
-    return nbt;
-  };
-  for (int vb = blockIdx.x; vb < nbt;) {
-  int tm, tn;
-  tile_coords<group_m<OCC>()>(vb, nbt, p.tiles_m, p.tiles_n, tm, tn);
-  const int m0 = tm * BM;
-  const int n0 = tn * BN;
-  // Persistent blocks: alternate rounds of an XCD's tiles (round = local index / workgroups per XCD) sweep K in
-  // opposite directions. The raster's consecutive rounds share their m-tiles' A rows, so a reversed round starts on
-  // the K range the previous round read last, which is still in the L2: 15 % fewer bytes fetched beyond the L2 at
-  // c1 (3.79 -> 3.23 GB), the same time. The int32 sums do not depend on the order; group-32's fp32 sum over the
-  // groups does (and its scale DMA follows kt), so it always sweeps forward.
-  const bool rev = PERSIST && !G32 && (((vb >> 3) / max(1, (int)(gridDim.x >> 3))) & 1);
 
   // Buffer resources based at the block's first row. Rows past M / N, and the DMA of a stage past the end of K
   // (offset kOOB), lie outside num_records: those loads read no memory.
@@ -903,9 +853,7 @@ void gemm_dma_kernel(const GemmArgs p) {
   }
   wait_dma<0>();     // the epilogue operands, and the out-of-range DMAs of the last iterations, have landed
   __syncthreads();   // every wave is done reading the ring: it becomes the output staging area
-  // the own-list claim of the next tile goes out now; its result is read after the epilogue, which covers its latency
-  int own = 0;
-  if (PERSIST && p.sched && wave == 0 && lane == 0) own = claim_own();
+  before_epilogue();
   if constexpr (ELDS) {
     // buffers of stages KT (rows) and KT + 1 (columns) hold the operands; staging in the NS - 2 others
     constexpr int kSpb = STAGE / Epi::kStageBytesL;
@@ -917,26 +865,121 @@ void gemm_dma_kernel(const GemmArgs p) {
     static_assert(ELDS || NW * Epi::kStageBytes <= NS * STAGE, "output staging must fit the LDS ring");
     epi.run(p, acc, nbase, mbase, lane, ring + wave * Epi::kStageBytes);
   }
-  if constexpr (PERSIST) {
+}
+
+// Bytes of LDS of a tile's ring and scale slots.
+template <int TI, int TJ, int WMW, int NS, int MODE>
+constexpr int tile_lds() {
+  constexpr int sb = MODE == kModeGroup32 ? 2 * 64 * TI * 4 : 0;
+  return NS * (64 * TI + 32 * TJ * WMW) * kBKd + (NS + 1) * sb;
+}
+
+// Ring of the quarter tiles (128 x 128 on 8 waves): 8 stages of 16 KB.
+constexpr int kQuarterStages = 8;
+
+template <int TI, int TJ, int WMW, int NS, int OCC, bool PACKED, int MODE, int LRS, int LRDT, int ODT, bool ACC = false>
+__global__ __attribute__((amdgpu_flat_work_group_size(128 * WMW, 128 * WMW),
+                          amdgpu_waves_per_eu(OCC * WMW / 2, OCC * WMW / 2)))
+void gemm_dma_kernel(const GemmArgs p) {
+  constexpr int BN = 64 * TI, BM = 32 * TJ * WMW, STAGE = (BN + BM) * kBKd;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[tile_lds<TI, TJ, WMW, NS, MODE>()];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nbt = p.tiles_m * p.tiles_n;
+  constexpr bool PERSIST = persistent_block<TI, TJ, WMW, NS, OCC, MODE, LRS, LRDT, ODT, ACC>();
+  if constexpr (!PERSIST) {
+    int tm, tn;
+    tile_coords<group_m<OCC>()>(blockIdx.x, nbt, p.tiles_m, p.tiles_n, tm, tn);
+    gemm_tile<TI, TJ, WMW, NS, OCC, PACKED, MODE, LRS, LRDT, ODT, ACC>(p, smem, lane, wave, tm * BM, tn * BN, false, [] {});
+    return;
+  } else {
+  // Persistent blocks (the 256 x 256 tile with its epilogue operands in the ring, no accumulate): one workgroup per
+  // CU loops over tiles, which takes the relaunch gap out of every tile after the first. XCD x's list holds its tiles in
+  // the order the launch-per-tile grid would give them (tile_coords: block id 8 li + x), so a workgroup stays on its
+  // XCD's tiles and the raster is unchanged. The first tile of workgroup b is entry b / 8 of list b % 8. After that,
+  // with a scheduling buffer (p.sched: 8 per-XCD claim counters and an exit count, zero at launch), a workgroup claims
+  // the next entry of its own XCD's list, and once that is empty it claims from the other XCDs' lists. The XCDs of one
+  // chip run the loop at different speeds (up to 5 % apart), so fixed shares finish up to 165 us apart at c1. Without
+  // the buffer it steps through its own list (a fixed share per workgroup).
+  //
+  // Tiles past a list's last whole round (a tile for every workgroup of the XCD) are handed out as four 128 x 128 quarters
+  // where the quarters are no more than the workgroups: a quarter takes about a third of a tile's time, so they end the
+  // product that much earlier (launch_dma sets whole_lo / whole_hi). Measured, start and now: M = 4352, K = 3072, N =
+  // 12288 (3.19 rounds) 163.7 and 158.7 us, 16640 x 3072 x 3072 (3.05) 171.4 and 157.6, 16640 x 12288 x 3072 538.8 and
+  // 495.5; where other XCDs' claims already cover the short round (65792 x 3072 x 3072, 12.05 rounds) the same. Two
+  // rounds of quarters lose: 4352 x 3072 x 9216 (2.39 rounds) 122.3 whole, 132.6 in quarters.
+  const int wgx = ((int)gridDim.x + 7) >> 3;   // workgroups per XCD (a grid smaller than the tiles is a multiple of 8)
+  const int x0 = blockIdx.x & 7;
+  auto xcd_cnt = [&](int x) { return (nbt >> 3) + (x < (nbt & 7) ? 1 : 0); };
+  auto xcd_whole = [&](int x) { return x < (nbt & 7) ? p.whole_hi : p.whole_lo; };   // tiles of list x that go out whole
+  auto xcd_entries = [&](int x) { return 4 * xcd_cnt(x) - 3 * xcd_whole(x); };
+  // Claims (lane 0 of wave 0). Part 1, issued before the epilogue so that the atomic's round trip overlaps it: the next
+  // entry of the own list.
+  auto claim_own = [&]() -> int { return atomicAdd(p.sched + x0, 1) + wgx; };
+  // Part 2, after the epilogue: the own entry if the list still had one, else the other 7 lists in a rotated order, so
+  // that stealers spread over the victims. Without a scheduling buffer, the fixed share. 8 li + x, or -1: nothing left.
+  auto claim_rest = [&](int vb, int own) -> int {
+    if (!p.sched) return (vb >> 3) + wgx < xcd_entries(x0) ? vb + 8 * wgx : -1;
+    if (own < xcd_entries(x0)) return (own << 3) | x0;
+    const int rot = blockIdx.x >> 3;
+    for (int k = 1; k < 8; ++k) {
+      const int x = (x0 + 1 + (k - 1 + rot) % 7) & 7;
+      const int li = atomicAdd(p.sched + x, 1) + wgx;
+      if (li < xcd_entries(x)) return (li << 3) | x;
+    }
+    return -1;
+  };
+  int vb = blockIdx.x;
+  int own = 0;
+  while (vb >= 0 && (vb >> 3) < xcd_whole(vb & 7)) {
+    int tm, tn;
+    tile_coords<group_m<OCC>()>(vb, nbt, p.tiles_m, p.tiles_n, tm, tn);
+    // Alternate rounds of an XCD's tiles sweep K in opposite directions. The raster's consecutive rounds share their
+    // m-tiles' A rows, so a reversed round starts on the K range the previous round read last, which is still in the L2:
+    // 15 % fewer bytes fetched beyond the L2 at c1 (3.79 -> 3.23 GB), the same time. The int32 sums do not depend on the
+    // order.
+    const bool rev = ((vb >> 3) / wgx) & 1;
+    gemm_tile<TI, TJ, WMW, NS, OCC, PACKED, MODE, LRS, LRDT, ODT, ACC>(p, smem, lane, wave, tm * BM, tn * BN, rev, [&] {
+      // the own-list claim goes out now; its result is read after the epilogue, which covers its latency
+      if (p.sched && wave == 0 && lane == 0) own = claim_own();
+    });
     // The next tile reaches every wave through the last 4 bytes of the row-operand buffer: its last DMA slot is
-    // past the row operands (kRowSlots < 32), so the epilogue never reads it, and the next tile's DMA overwrites it
-    // only after the second barrier.
-    static_assert(kRowSlots < NW * (DW + DA), "the row buffer's last slot holds no epilogue operand");
-    int* const slot = reinterpret_cast<int*>(ring + (KT % NS) * STAGE + STAGE - 4);
+    // past the row operands, so the epilogue never reads it, and the next tile's DMA overwrites it only after the second
+    // barrier.
+    static_assert(2 + BM * LRS * 16 * 2 / 1024 < (BN + BM) / 16, "the row buffer's last slot holds no epilogue operand");
+    int* const slot = reinterpret_cast<int*>(smem + (p.K / kBKd % NS) * STAGE + STAGE - 4);
     if (wave == 0 && lane == 0) *slot = claim_rest(vb, own);
     lds_barrier();
-    vb = *slot;
+    vb = __builtin_amdgcn_readfirstlane(*slot);
     lds_barrier();   // every wave has read it, and is done with the staging area, before the next tile's DMA
-  } else {
-    vb = nbt;
   }
+  // Quarters (and a whole tile claimed from another XCD's list meanwhile, as its four quarters).
+  while (vb >= 0) {
+    const int x = vb & 7, whole = xcd_whole(x), li = vb >> 3, q = li - whole;
+    int tm, tn;
+    tile_coords<group_m<OCC>()>(((q < 0 ? li : whole + (q >> 2)) << 3) | x, nbt, p.tiles_m, p.tiles_n, tm, tn);
+    for (int u = q < 0 ? 0 : q & 3, e = q < 0 ? 4 : u + 1; u < e; ++u) {
+      const int m0 = tm * BM + (u >> 1) * (BM / 2), n0 = tn * BN + (u & 1) * (BN / 2);
+      if (m0 >= p.M || n0 >= p.N) continue;
+      gemm_tile<TI / 2, TJ / 2, WMW, kQuarterStages, OCC, PACKED, MODE, LRS, LRDT, ODT, ACC>(p, smem, lane, wave, m0, n0,
+                                                                                            false, [] {});
+      lds_barrier();   // every wave is done with the staging area
+    }
+    static_assert(tile_lds<TI / 2, TJ / 2, WMW, kQuarterStages, MODE>() + 4 <= sizeof(smem), "the slot lies past the ring");
+    int* const slot = reinterpret_cast<int*>(smem + sizeof(smem) - 4);
+    if (wave == 0 && lane == 0) *slot = claim_rest(vb, p.sched ? claim_own() : 0);
+    lds_barrier();
+    vb = __builtin_amdgcn_readfirstlane(*slot);
+    lds_barrier();
   }
   // The last workgroup out leaves the scheduling buffer as it found it (zero) for the caller's next launch.
-  if (PERSIST && p.sched && wave == 0 && lane == 0) {
+  if (p.sched && wave == 0 && lane == 0) {
     if (atomicAdd(p.sched + 8, 1) == (int)gridDim.x - 1) {
 #pragma unroll
       for (int x = 0; x < 9; ++x) atomicExch(p.sched + x, 0);
     }
+  }
   }
 }
 
@@ -1098,8 +1141,13 @@ int launch_dma(GemmArgs& a, hipStream_t stream) {
   a.sched = nullptr;
   if constexpr (persistent_block<TI, TJ, WMW, NS, OCC, MODE, LRS, LRDT, ODT, ACC>()) {
     // one workgroup per CU; each XCD's share of workgroups claims that XCD's tiles (see the kernel)
-    const int wg = persistent_workgroups(stream);
+    const int wg = persistent_workgroups(stream), lo = (int)(grid.x / 8);
+    a.whole_lo = lo;
+    a.whole_hi = lo + 1;
     if (wg > 0 && grid.x > (unsigned)wg) {
+      const int wgx = wg / 8;
+      a.whole_lo = 4 * (lo % wgx) <= wgx ? lo - lo % wgx : lo;
+      a.whole_hi = 4 * ((lo + 1) % wgx) <= wgx ? lo + 1 - (lo + 1) % wgx : lo + 1;
       grid.x = (unsigned)wg;
       a.sched = sched;
     }

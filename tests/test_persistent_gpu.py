@@ -206,3 +206,39 @@ def test_layer_call_fresh_workspace_and_graph(cuda):
         print(f"[persistent] layer call, graph replay {i}", flush=True)
         assert torch.equal(y_g, ref), f"replay {i}"
         assert torch.equal(y_e, ref), f"eager call beside replay {i}"
+
+
+# 256 x 256 tiles per XCD list over 32 workgroups: 33 and 34 (some lists one tile longer), quarters that hang over the
+# last rows (M % 256 = 56: the lower quarters are empty) and columns (N % 256 = 64), 40 tiles (8 over: the most that go
+# out in quarters) and 41 (whole again)
+@pytest.mark.parametrize("sched", [True, False])
+@pytest.mark.parametrize("lr,shape", [(32, (4152, 4096 + 64, 128)), (0, (5120, 4096, 192)), (16, (5248, 4096, 64)),
+                                      (0, (2560, 8192 + 192, 320))])
+def test_last_tiles_in_quarters(cuda, sched, lr, shape):
+    """Lists that end in a few tiles past a whole round hand those out as 128 x 128 quarters: every tile written, with
+    the bits of the one-tile-per-workgroup kernels, with claims and with fixed shares, scattered too."""
+    from pyraquant_amd import int8_exec as E
+
+    M, N, K = shape
+    P = _problem(cuda, 5 + lr, lr, shape)
+    ref = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+    for r0 in range(0, M, 256):
+        m = min(256, M - r0)
+        t = None if P["t"] is None else P["t"][r0:r0 + m]
+        E.int8_gemm_packed(P["ap"][r0 * K:], P["s_row"][r0:], P["wp"], P["s_w"], P["bias"], m, N, K, torch.bfloat16, t=t,
+                           l2t=P["l2t"], out=ref[r0:r0 + m])
+    buf = torch.zeros(9, dtype=torch.int32, device=cuda) if sched else None
+    L = __import__("pyraquant_amd._lib", fromlist=["load"])
+    lib = L.load()
+    idx = torch.randperm(M, generator=torch.Generator().manual_seed(3)).to(torch.int32).to(cuda)
+    for rows in (None, idx):
+        for i in range(2):
+            out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+            st = lib.pq_int8_gemm_packed(L.ptr(P["ap"]), L.ptr(P["wp"]), L.ptr(P["s_row"]), L.ptr(P["s_w"]), 0,
+                                         L.ptr(P["bias"]), L.ptr(P["t"]), lr, L.ptr(P["l2t"]), lr, L.PQ_BF16, L.ptr(out), N,
+                                         L.PQ_BF16, L.ptr(rows), M, M, N, K, L.ptr(buf), L.stream_of(cuda))
+            assert st == 0, lib.pq_last_error()
+            got = out if rows is None else out[rows.long()]
+            assert torch.equal(got, ref), (rows is not None, i)
+    if sched:
+        assert not buf.any()
