@@ -31,8 +31,8 @@
 // (one MFMA from zero) the VALU converts and fma's with s_w[g, n] into an fp32 accumulator held in VGPRs, groups in
 // order. The scales of each stage ride the DMA ring (dword LDS-DMA, a ring of NS + 1 slots of their own). That is
 // 16 converts + 16 FMAs per lane per MFMA (128 VALU cycles of a wave64 against 32 of the MFMA), so group-32 is
-// VALU-bound at a quarter of the INT8 MFMA rate; blocks are 128 x 128 at two workgroups per CU (128 x 64 for small
-// problems and with a low-rank term).
+// VALU-bound at a quarter of the INT8 MFMA rate; blocks are 128 x 128 at three workgroups per CU, or 128 x 64 at four
+// (two with a low-rank term).
 //
 // Workgroup ids are remapped so that each XCD (ids are dealt round-robin over the 8 XCDs) walks a contiguous
 // run of tiles, rasterised in groups of group_m() m-tiles for L2 reuse. Large 256 x 256 products run one persistent
@@ -118,7 +118,7 @@ __device__ __forceinline__ v16f lr_mfma(v4i a, v4i b, v16f c) {
 // NTS: output stores carry the non-temporal hint (streamed past the L2). The large blocks' outputs (c1: 1.6 GB per
 // launch) are never re-read by the kernel, and keeping them out of the L2 leaves it to the operand tiles (measured
 // 0.5-1.3 % faster at c1 / c2b in the layer step).
-template <int TI, int TJ, int MODE, int LRS, int LRDT, int ODT, int CB = 2, bool NTS = false, bool ACC = false>
+template <int TI, int TJ, int MODE, int LRS, int LRDT, int ODT, int CB = 2, bool NTS = false, bool ACC = false, int PADL = 16>
 struct Epilogue {
   // CB = 2: the column operands of weight tile i + 1 load while tile i is computed (one workgroup per CU);
   // CB = 1: loaded right before use (two workgroups per CU hide the latency and the register budget is halved).
@@ -186,8 +186,9 @@ struct Epilogue {
     const int line = b >> 6, ch = (b >> 4) & 3;
     return 2048 + line * 64 + ((ch ^ k64_swz(line & 15)) << 4);
   }
-  // Output staging of run_lds: 32 rows x 64 outputs (two weight tiles) per pass, rows padded by 16 bytes.
-  static constexpr int kPitchL = 128 + 16;
+  // Output staging of run_lds: 32 rows x 64 outputs (two weight tiles) per pass, rows padded by PADL bytes (0 where a
+  // three-stage ring has room for no more).
+  static constexpr int kPitchL = 128 + PADL;
   static constexpr int kStageBytesL = 32 * kPitchL;
 
   // nloc / mloc: the wave's first column / row inside the workgroup block; nbase / mbase: the same, global.
@@ -481,7 +482,7 @@ __device__ __forceinline__ void lds_barrier() {
 // stage each and the operand DMA slots of one stage, and the output staging the remaining NS - 2 buffers.
 template <int TI, int TJ, int WMW, int NS, int OCC, int MODE, int LRS, int LRDT, int ODT, bool ACC>
 constexpr bool epilogue_in_ring() {
-  using Epi = Epilogue<TI, TJ, MODE, LRS, LRDT, ODT, OCC * WMW == 2 ? 2 : 1, OCC == 1, ACC>;
+  using Epi = Epilogue<TI, TJ, MODE, LRS, LRDT, ODT, OCC * WMW == 2 ? 2 : 1, OCC == 1, ACC, OCC == 3 ? 0 : 16>;
   constexpr int NW = 2 * WMW, BN = 64 * TI, BM = 32 * TJ * WMW;
   constexpr int stage = (BN + BM) * kBKd, dma = (BN + BM) / 16;   // bytes and 1 KB DMA slots of a stage
   constexpr int lr = LRS * 16 * 2;                                // one low-rank row
@@ -518,7 +519,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   static_assert(DW * 16 * NW == BN && DA * 16 * NW == BM && DS * 256 * NW == SB, "DMA split over the waves");
   constexpr int DPW = DW + DA + DS;
   // Epilogue operands through the ring (run_lds): see epilogue_in_ring.
-  using Epi = Epilogue<TI, TJ, MODE, LRS, LRDT, ODT, OCC * WMW == 2 ? 2 : 1, OCC == 1, ACC>;
+  using Epi = Epilogue<TI, TJ, MODE, LRS, LRDT, ODT, OCC * WMW == 2 ? 2 : 1, OCC == 1, ACC, OCC == 3 ? 0 : 16>;
   constexpr int kLrBytes = LRS * 16 * 2;                       // one low-rank row
   constexpr int kRowSlots = 2 + BM * kLrBytes / 1024, kColSlots = 2 + BN * kLrBytes / 1024;
   constexpr bool ELDS = epilogue_in_ring<TI, TJ, WMW, NS, OCC, MODE, LRS, LRDT, ODT, ACC>();
@@ -534,6 +535,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   uint8_t* const ring = smem + SLOTS * SB;
   const int wn = wave & 1;
   const int wm = wave >> 1;
+  // (group-32 is bound by the VALU: a wave whose rows all lie past M leaves it to the others)
+  const bool no_rows = G32 && m0 + wm * (BM / WMW) >= p.M;
 
   // Buffer resources based at the block's first row. Rows past M / N, and the DMA of a stage past the end of K
   // (offset kOOB), lie outside num_records: those loads read no memory.
@@ -689,6 +692,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint8_t* smem, int 
   // n = wn BN / 2 + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4.
   auto mm = [&](const v4i (&f)[NF], int kt, int s) {
     if constexpr (G32 && LRS == 0) {
+      // (The branch also keeps the compiler from opening all tiles of a substep at once: 130 VGPRs instead of 180, which
+      // lets three waves share a SIMD. At two per SIMD it costs 3 %, so it stays out there.)
+      if (OCC == 3 && no_rows) return;
       // Transposed tiles (no low-rank term to line up with): the activation fragment is the MFMA's first operand, so
       // lane l holds output column n = l % 32 of each tile and its 16 rows m; all 16 partials of a lane share one
       // scale s_w[g, n], one dword per weight tile and group instead of the 16-value stripe of the other layout.
@@ -890,7 +896,15 @@ void gemm_dma_kernel(const GemmArgs p) {
   constexpr bool PERSIST = persistent_block<TI, TJ, WMW, NS, OCC, MODE, LRS, LRDT, ODT, ACC>();
   if constexpr (!PERSIST) {
     int tm, tn;
-    tile_coords<group_m<OCC>()>(blockIdx.x, nbt, p.tiles_m, p.tiles_n, tm, tn);
+    // Group-32: the last row of tiles, where it is not full, goes to the XCDs in turn (left in the raster it would be one
+    // XCD's, at its end), and its waves without rows skip their products.
+    const int full = MODE == kModeGroup32 ? p.M / BM * p.tiles_n : nbt;
+    if ((int)blockIdx.x < full) {
+      tile_coords<group_m<OCC>()>(blockIdx.x, full, MODE == kModeGroup32 ? p.M / BM : p.tiles_m, p.tiles_n, tm, tn);
+    } else {
+      tm = p.tiles_m - 1;
+      tn = blockIdx.x - full;
+    }
     gemm_tile<TI, TJ, WMW, NS, OCC, PACKED, MODE, LRS, LRDT, ODT, ACC>(p, smem, lane, wave, tm * BM, tn * BN, false, [] {});
     return;
   } else {
@@ -1191,16 +1205,25 @@ inline bool big_tiles(const GemmArgs& a, hipStream_t stream) {
 template <bool PACKED, int MODE, int LRS, int LRDT, int ODT, bool ACC>
 int dispatch_tiles(GemmArgs& a, hipStream_t stream) {
   if constexpr (MODE == kModeGroup32) {
-    // fp32 accumulators live in VGPRs (the VALU rescales them every group): 128 x 128 blocks, two per CU; with
-    // fewer than 512 of them, 128 x 64 blocks (the VALU-bound kernel then spreads over twice the CUs: measured
-    // 1.2-1.5x faster at M = 2048 for the SDXL shapes, slower once the 128 x 128 blocks fill the chip). With a
-    // low-rank epilogue always 128 x 64: at 128 x 128 its slices of t and l2t push the kernel past its 256 VGPRs
-    // (5-49 spilled).
+    // fp32 accumulators live in VGPRs (the VALU rescales them every group): 128 x 128 blocks, three per CU, or 128 x 64
+    // blocks, four per CU. More waves per SIMD keep the VALU busy through each other's MFMAs, loads, first stages and
+    // epilogues: 16384 x 1280 x 5120 (M x K x N) 233.9 us in 128 x 128 blocks at two per CU, 223.5 at three; 65536 x 640 x
+    // 5120 540.6 and 501.1; 8202 x 640 x 5120 72.7 and 66.7. The kernel is bound by the VALU, so the time goes by the blocks
+    // on the fullest CU; a 128 x 64 block takes 5-10 % more than half a 128 x 128 one. 128 x 128 and 128 x 64: 8192 x 5120 x
+    // 1280 (640 blocks on 256 CUs: 3 rounds against 5 half ones) 124.6 and 114.9 us, 10000 x 1280 x 1280 (790: 4 against 7
+    // halves) 47.5 and 42.8, 9000 x 1280 x 1280 (710: 3 against 6) 36.3 and 37.5, 16384 x 5120 x 1280 (1280) 210.4 and
+    // 220.0. Up to two blocks per CU the smaller ones: 8192 x 2560 x 640 (320) 45.4 and 36.2, 1024 x 1280 x 1280 (80) 20.1
+    // and 12.6, 6400 x 1280 x 1280 (500) 26.7 and 26.8. With a low-rank epilogue always 128 x 64 at two per CU: at 128 x 128
+    // its slices of t and l2t push the kernel past its 256 VGPRs (5-49 spilled).
     if constexpr (LRS > 0) {
       return launch_dma<2, 1, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     } else {
-      if (small_blocks(a) < 512) return launch_dma<2, 1, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
-      return launch_dma<2, 2, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
+      const int64_t wg = persistent_workgroups(stream), cus = wg > 0 ? wg : 256, blocks = small_blocks(a);
+      const int64_t halves = (int64_t)((a.M + 63) / 64) * ((a.N + 127) / 128);
+      const int64_t t128 = 2 * ((blocks + cus - 1) / cus), t64 = (halves + cus - 1) / cus;   // on the fullest CU
+      if (blocks <= 2 * cus || 10 * t128 > 11 * t64)
+        return launch_dma<2, 1, 2, 4, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
+      return launch_dma<2, 2, 2, 3, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     }
   } else {
     // so few outputs that 64 x 32 or 64 x 64 blocks fit the CUs at once: K split over each block's waves

@@ -183,3 +183,40 @@ def test_gemm_rejects_bad_shapes(cuda):
     a, w = _codes(16, 96, 64, 1, cuda)        # N % 64 != 0
     with pytest.raises(AssertionError):
         E.int8_gemm_fused(a, torch.ones(16, device=cuda), w, torch.ones(96, device=cuda), None, torch.bfloat16)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    # 128 x 64 blocks: up to two 128 x 128 per CU, and above where their last round is the fuller
+    (1, 128, 64), (65, 192, 96 * 2), (2048, 640, 128), (8192, 1280, 64), (10000, 1280, 64),
+    # 128 x 128 blocks at three per CU: 513 blocks, ragged rows (10, 33 and 65 of the last 128, with waves that have
+    # none) and a half-filled last column
+    (65536, 256, 64), (8202, 5120, 192), (16417, 1280, 128), (9025, 1472, 320)])
+@pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.float16, False)])
+def test_group32_blocks(cuda, M, N, K, dtype, bias):
+    """Both group-32 blocks at their limits: each output bit for bit the fp32 chain fma(s_w[g], partial_g, ..) over the
+    groups in order, times s_row, plus bias, rounded once (fma evaluated in float64, whose single rounding to fp32 is
+    exact here: a 24-bit scale times a 20-bit partial and a 24-bit sum fit 53 bits unless the sum cancels far below its
+    terms; those few elements may differ by one rounding of the 16-bit type)."""
+    from pyraquant_amd import int8_exec as E
+
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    a = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device=cuda)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=cuda)
+    sr = torch.rand(M, generator=g, device=cuda) * 0.05 + 1e-3
+    sw = torch.rand(K // 32, N, generator=g, device=cuda) * 2e-4 + 1e-5
+    b = torch.randn(N, generator=g, device=cuda) * 0.01 if bias else None
+    out = E.int8_gemm_packed(E.pack_k64(a), sr, E.pack_k64(w), sw, b, M, N, K, dtype, group=32)
+    rows = torch.cat([torch.arange(min(M, 96)), torch.randint(0, M, (96,)), torch.arange(max(0, M - 140), M)]).unique()
+    rows = rows.to(cuda)
+    acc = torch.zeros(rows.numel(), N, dtype=torch.float32, device=cuda)
+    for j in range(K // 32):
+        part = a[rows, 32 * j:32 * j + 32].double() @ w[:, 32 * j:32 * j + 32].double().t()
+        acc = (part * sw[j].double() + acc.double()).float()
+    y = acc * sr[rows][:, None]
+    if bias:
+        y = y + b
+    ref = y.to(dtype)
+    diff = out[rows].view(torch.int16) != ref.view(torch.int16)
+    assert float(diff.float().mean()) <= 1e-5
+    eps = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    assert bool(((out[rows].float() - ref.float()).abs() <= eps * ref.float().abs() + 1e-6).all())
