@@ -109,6 +109,17 @@ def load():
     return _lib
 
 
+def load_direct():
+    """The eager layer call of _direct.so (csrc/pq_torch.cpp): linear(instance_dict, buffers, x)."""
+    load()
+    try:
+        from . import _direct
+    except ImportError as e:
+        raise LibraryMissing(f"pyraquant_amd/_direct.so is not built or does not load ({e}); run "
+                             "`python -m pyraquant_amd.build`") from e
+    return _direct.linear
+
+
 def check(status: int, what: str) -> None:
     if status == PQ_OK:
         return

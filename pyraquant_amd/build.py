@@ -1,6 +1,7 @@
-"""Build libpqint8.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Build libpqint8.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc, and _direct.so (the eager layer call, a CPython
+extension over torch's C++ API and the library) with the host compiler.
 
-    python -m pyraquant_amd.build          # compiles every csrc/*.hip, links pyraquant_amd/libpqint8.so
+    python -m pyraquant_amd.build          # compiles every csrc/*.hip, links pyraquant_amd/libpqint8.so, and _direct.so
 
 Flags: gfx950 only; -ffp-contract=off so the fp32 epilogue follows source order (multiply, then add, as
 the reference's epilogue is written); correctly rounded fp32 division (the quantizer's codes depend on
@@ -12,12 +13,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libpqint8.so")
+DIRECT_PATH = os.path.join(HERE, "_direct.so")
 ARCH = "gfx950"
 
 HIP_FLAGS = [
@@ -84,6 +87,34 @@ def _write_resources(rows: list) -> None:
     os.replace(RESOURCES_PATH + ".tmp", RESOURCES_PATH)
 
 
+def _compile_direct(obj: str) -> None:
+    """csrc/pq_torch.cpp (host code) -> obj."""
+    import torch
+    from torch.utils import cpp_extension
+
+    includes = [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in includes), "-c", os.path.join(CSRC, "pq_torch.cpp"), "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on pq_torch.cpp:\n{r.stdout}{r.stderr}")
+
+
+def _link_direct(obj: str) -> None:
+    """_direct.so against torch's libraries (loaded with torch) and libpqint8.so beside it."""
+    import torch
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = DIRECT_PATH + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, obj, f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+           f"-L{HERE}", "-l:libpqint8.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"linking _direct.so failed:\n{r.stdout}{r.stderr}")
+    os.replace(tmp, DIRECT_PATH)
+
+
 def build(verbose: bool = False) -> str:
     """Compile every csrc/*.hip for gfx950 and link libpqint8.so (always recompiles); record each kernel's registers
     and spills in kernel_resources.tsv."""
@@ -105,18 +136,22 @@ def build(verbose: bool = False) -> str:
                 print(msg, file=sys.stderr)
             return obj, _parse_resources(text)
 
-        with ThreadPoolExecutor(max_workers=min(4, len(srcs))) as ex:
+        direct_obj = os.path.join(tmp, "pq_torch.o")
+        with ThreadPoolExecutor(max_workers=min(5, len(srcs) + 1)) as ex:
+            direct = ex.submit(_compile_direct, direct_obj)
             done = list(ex.map(compile_one, srcs))
+            direct.result()
         objs = [o for o, _ in done]
         for _, rows in done:
             resources.extend(rows)
         _write_resources(resources)
         out_tmp = LIB_PATH + ".tmp"
-        cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", out_tmp, *objs]
+        cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,-soname,libpqint8.so", "-o", out_tmp, *objs]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stdout}{r.stderr}")
         os.replace(out_tmp, LIB_PATH)
+        _link_direct(direct_obj)
     return LIB_PATH
 
 

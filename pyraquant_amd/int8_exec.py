@@ -221,7 +221,14 @@ def int8_gemm_i32(xq: torch.Tensor, w_int8: torch.Tensor) -> torch.Tensor:
 # Int8Linear.forward's direct path (one workspace allocation, raw pointers); False routes every call through the
 # general wrappers (same kernels, same bits).
 DIRECT_CALLS = True
+_direct_linear = None   # _direct.so's layer call, loaded at the first use
 _DIRECT_DTYPES = {torch.bfloat16: _lib.PQ_BF16, torch.float16: _lib.PQ_F16}
+
+
+def _load_direct():
+    global _direct_linear
+    _direct_linear = _lib.load_direct()
+    return _direct_linear
 
 
 def _raw_stream(dev: torch.device) -> int:
@@ -622,10 +629,16 @@ class Int8Linear(nn.Module):
         rounded as torch's 16-bit ``out + y`` rounds it: a Linear split along its input sums its halves this way."""
         if accumulate:
             assert out is not None, "accumulate=True adds into out="
-        if row_idx is None and out is None and out_row_idx is None and self.weight_packed is not None and DIRECT_CALLS:
-            y = self._forward_direct(x)
+        if row_idx is None and out is None and out_row_idx is None and DIRECT_CALLS:
+            y = (_direct_linear or _load_direct())(self.__dict__, self._buffers, x)   # no low-rank branch: native
             if y is not None:
+                if type(y) is int:
+                    _lib.check(y, "int8_linear")
                 return y
+            if self.weight_packed is not None:
+                y = self._forward_direct(x)
+                if y is not None:
+                    return y
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
         if x2.stride(1) != 1:
