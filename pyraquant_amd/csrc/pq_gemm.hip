@@ -1183,7 +1183,8 @@ int launch_ksplit(GemmArgs& a, hipStream_t stream) {
 inline int64_t small_blocks(const GemmArgs& a) { return (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128); }
 
 // Tile choice of the LDS-DMA kernel: 256 x 256 blocks of 8 waves at one workgroup per CU, or 128 x 128 blocks of 4
-// waves at two per CU (or 128 x 64 when even those are too few to fill the chip).
+// waves at two per CU (128 x 64 when even those are too few to fill the chip; 128 x 256 of 8 waves in between: see
+// dispatch_tiles).
 // * Large problems (at least 1024 blocks of 256 x 128) take 256 x 256 blocks: a third less LDS-DMA traffic per MFMA
 //   than two 256 x 128 workgroups of 4 waves (measured in the layer's back-to-back step, interleaved on one box: 2 %
 //   faster at K = 3072, 6 % at K = 12288).
@@ -1237,6 +1238,14 @@ int dispatch_tiles(GemmArgs& a, hipStream_t stream) {
       if ((a.M + 63) / 64 * bn <= cus) return launch_ksplit<2, 2, 4, 4, LRS, ODT, ACC>(a, stream);
     }
     if (big_tiles(a, stream)) return launch_dma<4, 2, 4, 1, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
+    // More 128 x 128 blocks than CUs, but blocks twice as tall (8 waves, the ping-pong loop) all fit at once: one
+    // of them takes less than the two blocks it replaces do sharing a CU. M x K x N, 128 x 128 and 128 x 256: 2048 x 3072 x
+    // 3072 29.1 and 24.4 us, 512 x 3072 x 12288 28.9 and 24.8, 4096 x 2560 x 1280 22.1 and 20.0, 4096 x 640 x 1280 11.0
+    // and 10.0. With one 128 x 128 block per CU or less they lose (2048 x 3072 x 2048 17.8 and 22.0), and in a second round
+    // (2700 x 3072 x 3072 35.9 and 44.2).
+    const int64_t wgs = persistent_workgroups(stream);
+    if (small_blocks(a) > wgs && (int64_t)((a.M + 255) / 256) * ((a.N + 127) / 128) <= wgs)
+      return launch_dma<2, 2, 4, 1, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     // fewer 128 x 128 blocks than half the CUs: 128 x 64 blocks (measured 1.3x faster at 80 blocks, even at 160)
     if (small_blocks(a) < 128) return launch_dma<2, 1, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     return launch_dma<2, 2, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);

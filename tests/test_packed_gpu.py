@@ -383,3 +383,37 @@ def test_few_blocks_split_k(cuda, M, K, N, R, dtype, scatter, accumulate):
     E.int8_gemm_packed(E.pack_k64(a), sr, E.pack_k64(w), sw, bias, M, N, K, dtype, t=t, l2t=l2t, out=canvas,
                        out_row_idx=idx, accumulate=accumulate)
     assert torch.equal(canvas.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,K,N", [(2048, 64, 3072), (2049, 128, 2304), (512, 576, 9216), (2160, 320, 3008), (4352, 128, 1280)])
+@pytest.mark.parametrize("R,accumulate", [(0, False), (0, True), (16, False), (32, False), (64, False), (64, True)])
+def test_tall_blocks(cuda, M, K, N, R, accumulate):
+    """128 x 256 blocks (more 128 x 128 blocks than CUs, but no more tall ones): K of 1, 2, 5 and 9 stages against the
+    ring, a last block of one row, a last column half filled, every rank and the accumulate mode, from packed and
+    row-major operands; the whole-number sums against an exact product, the outputs against 128 rows at a time, which
+    take other blocks, bit for bit."""
+    from pyraquant_amd import int8_exec as E
+
+    g = torch.Generator(device=cuda).manual_seed(M + K + N + R)
+    a = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device=cuda)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=cuda)
+    sr = torch.rand(M, generator=g, device=cuda) * 0.05 + 1e-3
+    sw = torch.rand(N, generator=g, device=cuda) * 2e-4 + 1e-5
+    b = torch.randn(N, generator=g, device=cuda) * 0.01
+    t = (torch.randn(M, R, generator=g, device=cuda) * 0.5).bfloat16() if R else None
+    l2t = (torch.randn(N, R, generator=g, device=cuda) * 0.02).bfloat16() if R else None
+    base = torch.randn(M, N, generator=g, device=cuda).bfloat16()
+    ap, wp = E.pack_k64(a), E.pack_k64(w)
+    y = E.int8_gemm_packed(ap, sr, wp, sw, b, M, N, K, torch.bfloat16, t=t, l2t=l2t,
+                           out=base.clone() if accumulate else None, accumulate=accumulate)
+    ref = base.clone()
+    for r0 in range(0, M, 128):
+        m = min(128, M - r0)
+        E.int8_gemm_packed(ap[r0 * K:], sr[r0:], wp, sw, b, m, N, K, torch.bfloat16, t=None if t is None else t[r0:r0 + m],
+                           l2t=l2t, out=ref[r0:r0 + m], accumulate=accumulate)
+    assert torch.equal(y, ref)
+    if not accumulate:
+        assert torch.equal(E._gemm(a, sr, w, sw, 0, b, t, l2t, torch.bfloat16), ref)
+    if R == 0 and not accumulate:
+        exact = (a.double() @ w.double().t()) * (sr[:, None] * sw[None, :]).double() + b.double()
+        assert bool(((y.double() - exact).abs() <= exact.abs() * 2.0 ** -8 + 1e-6).all())
