@@ -16,7 +16,8 @@
 // epilogue reads the accumulators in place, with no v_accvgpr_read copies). Large problems, and those whose 256 x 256
 // blocks all fit on the CUs at once while their 128 x 128 blocks would not, run 256 x 256 blocks of 8 waves at one
 // workgroup per CU (128 accumulators per wave, two waves per SIMD); smaller ones 128 x 128 blocks of 4 waves at two
-// workgroups per CU, or 128 x 64 when the 128 x 128 blocks are too few to fill the chip.
+// workgroups per CU, 128 x 256 of 8 waves where those fit at once and 128 x 128 ones would not, or 128 x 64 when the
+// 128 x 128 blocks are too few to fill the chip. Products of few blocks run gemm_ksplit_kernel.
 // K advances in stages of 64 bytes through a ring of NS LDS stages (5 x 32 KB for the 256 x 256 block) filled by
 // LDS-DMA buffer loads (buffer_load_dwordx4 ... lds): no VGPR staging, no ds_write, and NS - 1 stages of
 // prefetch in flight to cover L2 / MALL latency. One DMA instruction fills 1 KB = 16 LDS rows of 64 bytes;

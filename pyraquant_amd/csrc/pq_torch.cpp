@@ -4,10 +4,10 @@
 //
 // One call takes the place of the checks, the two allocations and the twenty-argument foreign call of
 // Int8Linear._forward_direct: an eager layer of few rows (one launch) costs the host 5.0 us, 14.2 before (two launches,
-// 5.5 us, and the rest Python and the foreign call). It looks its tensors up and checks them on every call; nothing is kept between calls. It takes layers without a low-rank
-// branch, whose tensors and x are plain torch tensors in the state the kernels read; for everything else it returns
-// None and the Python paths decide, as they do without it. Results, allocations (torch's caching allocator, on the
-// current stream) and refusals are those of the Python path.
+// 5.5 us, and the rest Python and the foreign call). It looks its tensors up and checks them on every call; nothing is
+// kept between calls. It takes layers without a low-rank branch, whose tensors and x are plain torch tensors in the state
+// the kernels read; for everything else it returns None and the Python paths decide, as they do without it. Results,
+// allocations (torch's caching allocator, on the current stream) and refusals are those of the Python path.
 #include <Python.h>
 
 #include <ATen/ops/empty.h>

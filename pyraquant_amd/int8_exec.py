@@ -218,8 +218,8 @@ def int8_gemm_i32(xq: torch.Tensor, w_int8: torch.Tensor) -> torch.Tensor:
 
 
 # --------------------------------------------------------------------------- packed K64 layer path
-# Int8Linear.forward's direct path (one workspace allocation, raw pointers); False routes every call through the
-# general wrappers (same kernels, same bits).
+# Int8Linear.forward's direct paths: the native call of _direct.so (layers without a low-rank branch), and one C call over
+# raw pointers for the rest; False routes every call through the general wrappers (same bits).
 DIRECT_CALLS = True
 _direct_linear = None   # _direct.so's layer call, loaded at the first use
 _DIRECT_DTYPES = {torch.bfloat16: _lib.PQ_BF16, torch.float16: _lib.PQ_F16}
@@ -584,11 +584,10 @@ class Int8Linear(nn.Module):
         return tuple(map(id, src)), src, dev, code, R, args
 
     def _forward_direct(self, x: torch.Tensor) -> Optional[torch.Tensor]:
-        """The common layer call (no routing arguments, packed weights) with the host work cut to one C call,
-        pq_int8_linear: codes, scales and t share one workspace allocation, operands go as raw pointers, the stream
+        """The common layer call (no routing arguments, packed weights) where the native call does not take it (a
+        low-rank branch, or tensors that are not plain), with the host work cut to one C call, pq_int8_linear: codes, scales and t share one workspace allocation, operands go as raw pointers, the stream
         is the raw current stream. What depends on the module alone (the checks of its buffers and their pointers)
-        is kept per input dtype and checked by identity on every call. Same kernels and arguments as the general
-        path, so the same bits; returns None when a precondition of this path does not hold."""
+        is kept per input dtype and checked by identity on every call. Same bits as the general path; returns None when a precondition of this path does not hold."""
         dt = x.dtype
         src = self._direct_sources()
         plans = self.__dict__.setdefault("_direct_plans", {})
