@@ -32,8 +32,8 @@
 // (one MFMA from zero) the VALU converts and fma's with s_w[g, n] into an fp32 accumulator held in VGPRs, groups in
 // order. The scales of each stage ride the DMA ring (dword LDS-DMA, a ring of NS + 1 slots of their own). That is
 // 16 converts + 16 FMAs per lane per MFMA (128 VALU cycles of a wave64 against 32 of the MFMA), so group-32 is
-// VALU-bound at a quarter of the INT8 MFMA rate; blocks are 128 x 128 at three workgroups per CU, or 128 x 64 at four
-// (two with a low-rank term).
+// VALU-bound at a quarter of the INT8 MFMA rate; blocks are 128 x 128 at three workgroups per CU, 128 x 64 at four (two
+// with a low-rank term), or 64 x 32 of two waves for few outputs.
 //
 // Workgroup ids are remapped so that each XCD (ids are dealt round-robin over the 8 XCDs) walks a contiguous
 // run of tiles, rasterised in groups of group_m() m-tiles for L2 reuse. Large 256 x 256 products run one persistent
@@ -1222,6 +1222,14 @@ int dispatch_tiles(GemmArgs& a, hipStream_t stream) {
     } else {
       const int64_t wg = persistent_workgroups(stream), cus = wg > 0 ? wg : 256, blocks = small_blocks(a);
       const int64_t halves = (int64_t)((a.M + 63) / 64) * ((a.N + 127) / 128);
+      // Few outputs: 64 x 32 blocks of two waves, one tile each, up to five per CU. A wave's groups run one after another
+      // (product, convert, fma), so with so few waves the time goes by the tiles of the busiest wave, which are half
+      // those of a 128 x 64 block's wave, and the finer blocks fill the CUs more evenly. 128 x 64 and 64 x 32: 77 x 5120 x
+      // 1280 (60 blocks) 34.8 and 24.9 us, 512 x 5120 x 1280 35.3 and 26.1, 1536 x 5120 x 1280 (960) 35.5 and 31.8, 2048 x
+      // 2560 x 640 19.7 and 15.6, 2048 x 5120 x 1280 (1280) 44.8 and 43.5; past five per CU they lose: 2200 x 5120 x 1280
+      // (1380) 45.2 and 51.3, 512 x 1280 x 10240 (2560) 22.5 and 25.0.
+      if ((int64_t)((a.M + 31) / 32) * ((a.N + 63) / 64) <= 5 * cus)
+        return launch_dma<1, 1, 1, 8, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
       const int64_t t128 = 2 * ((blocks + cus - 1) / cus), t64 = (halves + cus - 1) / cus;   // on the fullest CU
       if (blocks <= 2 * cus || 10 * t128 > 11 * t64)
         return launch_dma<2, 1, 2, 4, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);

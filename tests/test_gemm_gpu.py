@@ -220,3 +220,42 @@ def test_group32_blocks(cuda, M, N, K, dtype, bias):
     assert float(diff.float().mean()) <= 1e-5
     eps = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
     assert bool(((out[rows].float() - ref.float()).abs() <= eps * ref.float().abs() + 1e-6).all())
+
+
+@pytest.mark.parametrize("M,N,K", [
+    # 64 x 32 blocks: one row, one past a block's 32, rows that leave the second 16 of a block empty, one column block,
+    # and the last sizes with five per CU (2048 x 1280) before the 128 x 64 blocks
+    (1, 64, 64), (33, 192, 128), (80, 64, 320), (154, 1280, 2048), (2048, 1280, 128), (2049, 1280, 128)])
+@pytest.mark.parametrize("packed", [True, False])
+def test_group32_few_blocks(cuda, M, N, K, packed):
+    """The scattered output of a group-32 product of few blocks: its rows are those of the unscattered one, bit for bit
+    the fp32 chain over the groups (as test_group32_blocks), and the canvas's other rows keep what they held."""
+    from pyraquant_amd import int8_exec as E
+
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    a = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device=cuda)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=cuda)
+    sr = torch.rand(M, generator=g, device=cuda) * 0.05 + 1e-3
+    sw = torch.rand(K // 32, N, generator=g, device=cuda) * 2e-4 + 1e-5
+    b = torch.randn(N, generator=g, device=cuda) * 0.01
+    idx = torch.randperm(M + 7, generator=g, device=cuda)[:M].to(torch.int32)
+
+    def run(**kw):
+        if packed:
+            return E.int8_gemm_packed(E.pack_k64(a), sr, E.pack_k64(w), sw, b, M, N, K, torch.float16, group=32, **kw)
+        return E._gemm(a, sr, w, sw, 32, b, None, None, torch.float16, **kw)
+
+    canvas = torch.full((M + 7, N), 3.0, dtype=torch.float16, device=cuda)
+    run(out=canvas, out_row_idx=idx)
+    y = run()
+    assert torch.equal(canvas[idx.long()], y)
+    rest = torch.ones(M + 7, dtype=torch.bool, device=cuda)
+    rest[idx.long()] = False
+    assert bool((canvas[rest] == 3.0).all())
+    acc = torch.zeros(M, N, dtype=torch.float32, device=cuda)
+    for j in range(K // 32):
+        part = a[:, 32 * j:32 * j + 32].double() @ w[:, 32 * j:32 * j + 32].double().t()
+        acc = (part * sw[j].double() + acc.double()).float()
+    ref = (acc * sr[:, None] + b).to(torch.float16)
+    assert float((y.view(torch.int16) != ref.view(torch.int16)).float().mean()) <= 1e-5
+    assert bool(((y.float() - ref.float()).abs() <= 2.0 ** -10 * ref.float().abs() + 1e-6).all())
