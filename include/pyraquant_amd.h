@@ -85,8 +85,11 @@ const char* pq_last_error(void);
  * which is the reference's torch restatement (deploy/int8_exec.py:508-509). q is [M, K] contiguous.
  * x has x_rows rows (x_rows >= M without row_idx). A row_idx entry outside [0, x_rows) reads as a row of zeros
  * (codes 0, s = fl(1e-8) / 127) instead of memory past x; torch's index ops would raise there.
- * Inputs must be finite. Any K >= 1 and ldx >= K are accepted; 16-byte aligned x with ldx % 8 == 0 and
- * K % 8 == 0 takes the vectorised kernel, anything else a per-element kernel with the same results.
+ * Inputs should be finite. A row that is not still has codes in [-127, 127], the same in every kernel: infinite and NaN
+ * elements have code 0; the scale of a row with a NaN is that of a = 1e-8f and its finite elements have the codes above;
+ * without a NaN, the scale of a row with an infinity is infinite and its codes are 0.
+ * Any K >= 1 and ldx >= K are accepted; 16-byte aligned x with ldx % 8 == 0 and K % 8 == 0 takes the vectorised kernel,
+ * anything else a per-element kernel with the same results.
  */
 int pq_quant_rows(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, int64_t x_rows,
                   const int32_t* row_idx, int8_t* q, float* s, hipStream_t stream);

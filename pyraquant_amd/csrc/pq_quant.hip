@@ -16,6 +16,10 @@
 // low byte (round to nearest even; |q| < 2^22). Four instructions per element. A test for near ties with the division
 // beside it was as many, and its code, repeated for every chunk of a row, was what bound the kernels: 1.7 KB per
 // chunk, up to 84 KB in a kernel against the 64 KB instruction cache that two CUs share.
+//
+// Rows that are not finite (callers owe finite ones; the codes stay in [-127, 127] all the same, and every kernel gives
+// the same): an infinite or NaN element has code 0; the others of a row with an infinity have code 0, of a row with a
+// NaN, whose scale is the floor's, clamp(rint(x / s)) as ever (see saturate_nan_row).
 #include "pq_common.h"
 
 #include <algorithm>
@@ -56,6 +60,52 @@ __device__ __forceinline__ v2u quant_chunk(v4u v, float s, float rc) {
     m[i] = __builtin_fmaf(__builtin_fmaf(-q0, s, f), rc, q0) + kMagic;
   }
   return v2u{low_bytes4(m[0], m[1], m[2], m[3]), low_bytes4(m[4], m[5], m[6], m[7])};
+}
+
+// ---- rows with a NaN ---------------------------------------------------------------------------------------------
+// fmaxf takes the number, so the scale of such a row is the floor's and |x / s| reaches 1e49, where q + 1.5 * 2^23 holds
+// no code in its low byte. Its finite elements are clamped, still as 16-bit values, to the smallest magnitude whose code
+// is 127: the codes are those of clamp(rint(x / s)). NaN and infinite elements stay as they are (low byte 0; and a NaN
+// reaches every t of the row). A branch per row, taken for these rows alone, where a clamp per element would be a fifth
+// instruction for each; no case of 154 x 2048 x 1280 to 65536 x 12288 x 3072 changed by more than its runs differ.
+template <int DT>
+struct NanRow {
+  static constexpr uint32_t kInf = DT == PQ_BF16 ? 0x7f80u : 0x7c00u;   // magnitude bits above this: a NaN
+  // bf16: 0x1.58p-27, 127.15 floors. fp16: 2^-24, its smallest, which is 757 floors; the codes of the row then take a
+  // scale of their own, 2^-24 / 127.25 (not the scale of any finite row: those are multiples of 2^-24 by 127).
+  static constexpr uint16_t kLimit = DT == PQ_BF16 ? 0x322c : 0x0001;
+  static constexpr float kScale = 0x1p-24f / 127.25f;
+};
+
+// The elements of v whose row has a NaN (`nan`: a lane's whole v is of one row) clamped as above, and the row's code scale.
+template <int DT, int N>
+__device__ __forceinline__ void saturate_nan_row(v4u (&v)[N], bool nan, float& sc, float& rc) {
+  using L = NanRow<DT>;
+  const us2 limit = {L::kLimit, L::kLimit}, inf = {(uint16_t)L::kInf, (uint16_t)L::kInf};
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    // (opaque: the compiler would otherwise keep the magnitudes of the row's maximum for this branch, at twice the registers)
+    asm volatile("" : "+v"(v[c]));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const us2 mag = __builtin_bit_cast(us2, v[c][e] & 0x7fff7fffu);
+      const us2 low = __builtin_elementwise_min(mag, limit);
+      const us2 out = {mag.x < inf.x ? low.x : mag.x, mag.y < inf.y ? low.y : mag.y};
+      if (nan) v[c][e] = (v[c][e] & 0x80008000u) | __builtin_bit_cast(uint32_t, out);
+    }
+  }
+  if constexpr (DT == PQ_F16) {
+    if (nan) {
+      sc = L::kScale;
+      rc = __fdiv_rn(1.0f, L::kScale);
+    }
+  }
+}
+
+// The scale a row reports, from the scale of its codes.
+template <int DT>
+__device__ __forceinline__ float row_scale(float sc) {
+  return DT == PQ_F16 && sc == NanRow<DT>::kScale ? __fdiv_rn(1e-8f, 127.0f) : sc;
 }
 
 // Maximum over the 64 lanes of a wave, for values below 2^31, in DPP row operations (no LDS round trip): quad_perm
@@ -141,8 +191,9 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(
   uint32_t mx = mx2.x > mx2.y ? mx2.x : mx2.y;
   mx = wave_max_u32(mx);
   const float a = fmaxf(absmax_from_bits<DT>(mx), 1e-8f);
-  const float sc = __fdiv_rn(a, 127.0f);
-  const float rc = __fdiv_rn(1.0f, sc);
+  float sc = __fdiv_rn(a, 127.0f);
+  float rc = __fdiv_rn(1.0f, sc);
+  if (__builtin_expect(mx > NanRow<DT>::kInf, 0)) saturate_nan_row<DT>(v, true, sc, rc);
   if constexpr (PARTS) {
     float tv = pv[0];
 #pragma unroll
@@ -164,7 +215,7 @@ __global__ __launch_bounds__(256) void quant_rows_vec_kernel(
       }
     }
   }
-  if (lane == 0) s[m] = sc;
+  if (lane == 0) s[m] = row_scale<DT>(sc);
 }
 
 // Per-element quantizer for unaligned rows or odd K: one wave per row, two sweeps over the row (a gathered source row
@@ -199,7 +250,8 @@ __global__ __launch_bounds__(256) void quant_rows_scalar_kernel(
   int8_t* __restrict__ qr = q + m * (int64_t)K;
   for (int k = lane; k < K; k += 64) {
     const float f = live ? lo16_to_f32<DT>(xr[k]) : 0.0f;
-    const int8_t code = (int8_t)(__float_as_uint(code_exact(f, sc)) & 0xffu);
+    const bool finite = fabsf(f) < __builtin_inff();
+    const int8_t code = finite ? (int8_t)(__float_as_uint(code_exact(f, sc)) & 0xffu) : (int8_t)0;
     if constexpr (PACKED) {
       q[k64_offset(m, k, K >> 6)] = code;
     } else {
@@ -738,8 +790,9 @@ __global__ __launch_bounds__(64 * W, 1) void quant_lowrank_kernel(
 #pragma unroll
     for (int w = 1; w < W; ++w) am = am > amax_l[w][r] ? am : amax_l[w][r];
     const float a = fmaxf(lo16_to_f32<DT>(am), 1e-8f);
-    const float sc = __fdiv_rn(a, 127.0f);
-    const float rc = __fdiv_rn(1.0f, sc);
+    float sc = __fdiv_rn(a, 127.0f);
+    float rc = __fdiv_rn(1.0f, sc);
+    if (__builtin_expect(__any(am > NanRow<DT>::kInf), 0)) saturate_nan_row<DT>(xv, am > NanRow<DT>::kInf, sc, rc);
     // codes: block c of the slice, chunk g of row m (padding rows past M quantize zeros to zero codes)
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -747,7 +800,7 @@ __global__ __launch_bounds__(64 * W, 1) void quant_lowrank_kernel(
       const v2u hi = quant_chunk<DT>(xv[2 * c + 1], sc, rc);
       *reinterpret_cast<v4u*>(qp + k64_offset(m, k0 + 64 * c + 16 * g, K / 64)) = v4u{lo.x, lo.y, hi.x, hi.y};
     }
-    if (wave == 0 && g == 0 && m < M) s[m] = sc;
+    if (wave == 0 && g == 0 && m < M) s[m] = row_scale<DT>(sc);
     // low rank: partial t over the slice
     v4f acc[2] = {v4f{}, v4f{}};
 #pragma unroll
@@ -946,6 +999,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
       const float a = fmaxf(absmax_from_bits<DT>(mx), 1e-8f);
       sc[rho] = __fdiv_rn(a, 127.0f);
       rc[rho] = __fdiv_rn(1.0f, sc[rho]);
+      if (__builtin_expect(mx > NanRow<DT>::kInf, 0)) saturate_nan_row<DT>(v[rho], true, sc[rho], rc[rho]);
     }
     // packed K64 rows of the batch: rows b BR .. b BR + BR - 1 are rows (b BR) % 16 .. of block row b BR / 16, this
     // wave's first row is row rb0 = (b BR) % 16 + RPW w of its block (k64_offset, split into the wave-uniform part
@@ -1012,7 +1066,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
     if (lane == 0) {
 #pragma unroll
       for (int rho = 0; rho < RPW; ++rho)
-        if (mrow[rho] < M) s[mrow[rho]] = sc[rho];
+        if (mrow[rho] < M) s[mrow[rho]] = row_scale<DT>(sc[rho]);
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_sched_barrier(0);
@@ -1164,14 +1218,15 @@ __global__ __launch_bounds__(64 * kSmallWaves) void linear_small_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) mx2 = __builtin_elementwise_max(mx2, __builtin_bit_cast(us2, v[h][c][e] & 0x7fff7fffu));
     const uint32_t mx = wave_max_u32(mx2.x > mx2.y ? mx2.x : mx2.y);
-    const float sc = __fdiv_rn(fmaxf(absmax_from_bits<DT>(mx), 1e-8f), 127.0f);
-    const float rc = __fdiv_rn(1.0f, sc);
+    float sc = __fdiv_rn(fmaxf(absmax_from_bits<DT>(mx), 1e-8f), 127.0f);
+    float rc = __fdiv_rn(1.0f, sc);
+    if (__builtin_expect(mx > NanRow<DT>::kInf, 0)) saturate_nan_row<DT>(v[h], true, sc, rc);
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
       const int idx = c * 64 + lane;
       if (idx < nvec) *reinterpret_cast<v2u*>(codes + k64_offset(2 * wave + h, idx * 8, KT)) = quant_chunk<DT>(v[h][c], sc, rc);
     }
-    if (lane == 0) srow[2 * wave + h] = sc;
+    if (lane == 0) srow[2 * wave + h] = row_scale<DT>(sc);
   }
   __syncthreads();
   v4i acc[NT];

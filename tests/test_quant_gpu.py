@@ -195,3 +195,92 @@ def test_quant_rows_every_mantissa_pair(oracle, cuda, dtype):
             assert (q.cpu().numpy() == qo).all() and (s.cpu().numpy() == so).all()
             qp, _ = E.quant_rows_packed(xc.to(cuda))
             assert torch.equal(qp, E.pack_k64(q))
+
+
+def _codes_of(x):
+    """Codes and scales of rows that need not be finite: a row with a NaN has the floor's scale, an infinite or NaN
+    element code 0, every other clamp(rint(x / s)) (on the CPU, IEEE divisions)."""
+    xf = x.float()
+    a = torch.where(xf.isnan().any(1), torch.zeros(()), xf.abs().nan_to_num(nan=0.0, posinf=float("inf")).amax(1))
+    s = a.clamp_min(1e-8) / 127
+    q = torch.where(xf.isfinite(), (xf / s[:, None]).round().clamp(-127, 127), torch.zeros(()))
+    return q.to(torch.int8), s
+
+
+def _not_finite(M, K, dtype, seed):
+    """Finite rows, and at `rows` ones with a NaN, an infinity or both beside elements of every magnitude."""
+    from pyraquant_amd.workloads import make_x
+
+    x = make_x(M, K, dtype, seed=seed)
+    g = torch.Generator().manual_seed(seed)
+    rows = sorted({0, 1, 2, 17 % M, M // 2, M - 3, M - 2, M - 1})
+    for i, r in enumerate(rows):
+        x[r] = torch.randint(-32768, 32768, (K,), generator=g).to(torch.int16).view(dtype).nan_to_num(0.0, 0.0, 0.0)
+        x[r, 3:19] = torch.tensor([1e-8, -1e-8, 1.01e-8, 1e-7, -1e-6, 1e-5, -1e-4, 1e-3, 0.5, 1.0, -1.0, 2.0, 0.0, -0.0, 64.0, 3e4])
+        if i % 3 < 2:
+            x[r, (5 * r + 40) % K] = float("nan")
+        if i % 3 > 0:
+            x[r, K - 1], x[r, 1] = float("inf"), -float("inf")
+    return x, rows
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K", [(24, 64), (24, 520), (40, 1280), (24, 3072), (24, 12288), (24, 16384), (24, 1003)])
+def test_rows_that_are_not_finite(cuda, dtype, M, K):
+    """Codes of rows with NaN and infinite elements: in [-127, 127] and the same in the vectorised kernel (K % 8 == 0),
+    its packed form, and the per-element kernel, which an unaligned view takes."""
+    from pyraquant_amd import int8_exec as E
+
+    x, _ = _not_finite(M, K, dtype, seed=K)
+    qo, so = _codes_of(x)
+    wide = torch.zeros(M, K + 8, dtype=dtype, device=cuda)
+    wide[:, 1:K + 1] = x.to(cuda)
+    for q, s in (E.quant_rows(x.to(cuda)), E.quant_rows(wide[:, 1:K + 1])):
+        assert torch.equal(s.cpu(), so)
+        assert torch.equal(q.cpu(), qo)
+    if K % 64 == 0:
+        qp, s = E.quant_rows_packed(x.to(cuda))
+        assert torch.equal(s.cpu(), so) and torch.equal(qp, E.pack_k64(qo.to(cuda)))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K", [(40, 1024), (40, 1280), (40, 2560), (40, 3072),             # one-pass kernel: 16, 4, 8 waves
+                                 (40, 4096), (40, 12288), (4120, 12288), (2072, 15360)])      # wide kernel, and its tail
+def test_rows_that_are_not_finite_lowrank(cuda, dtype, M, K):
+    """The fused quantizer + down-projection: the same codes, NaN in every column of t for a row with a NaN, and no
+    other row touched by it."""
+    from pyraquant_amd import int8_exec as E
+
+    x, rows = _not_finite(M, K, dtype, seed=K)
+    l1t = (torch.randn(32, K, generator=torch.Generator().manual_seed(1)) * 0.05).to(dtype).to(cuda)
+    clean = x.clone()
+    clean[rows] = 0
+    q0, s0, t0 = E.quant_rows_lowrank(clean.to(cuda), l1t)
+    q, s, t = E.quant_rows_lowrank(x.to(cuda), l1t)
+    qo, so = _codes_of(x)
+    assert torch.equal(s.cpu(), so) and torch.equal(q, E.pack_k64(qo.to(cuda)))
+    keep = torch.ones(M, dtype=torch.bool)
+    keep[rows] = False
+    assert torch.equal(t[keep.to(cuda)], t0[keep.to(cuda)])
+    assert t[x.isnan().any(1).to(cuda)].isnan().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [64, 1280, 2048, 4096])
+def test_rows_that_are_not_finite_small_layer(cuda, dtype, K):
+    """The layer as one kernel against quantizer and GEMM on such rows, with weights large enough to show their codes."""
+    from pyraquant_amd import int8_exec as E
+
+    M, N = 24, 128
+    x, rows = _not_finite(M, K, dtype, seed=K)
+    lin = torch.nn.Linear(K, N, bias=False, device=cuda)
+    with torch.no_grad():
+        lin.weight.mul_(1e8 / K ** 0.5)
+    m = E.Int8Linear(lin)
+    xc = x.to(cuda)
+    q, s = E.quant_rows_packed(xc)
+    y2 = E.int8_gemm_packed(q, s, m.weight_packed, m.w_scale, None, M, N, K, dtype)
+    y = m(xc)
+    assert torch.equal(y.isnan(), y2.isnan()) and torch.equal(y.nan_to_num(0.0), y2.nan_to_num(0.0))
+    nan_only = [r for r in rows if x[r].isnan().any()]
+    assert (y[nan_only].abs() > 1e-3).any(1).all()
