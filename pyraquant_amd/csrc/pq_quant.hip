@@ -981,9 +981,12 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void quant_lowrank_wide_kernel(
       }
       live[rho] = src_of(more ? bn : b, rho) >= 0;   // the batch whose loads xn starts
     }
+    // (fenced from each other too: slab 0's wait counts on its four instructions being the older ones, and the buffers are
+    // separate arrays, which the compiler may fill in any order)
     dma_l(0);
+    __builtin_amdgcn_sched_barrier(0);
     dma_l(1);
-    __builtin_amdgcn_sched_barrier(0);   // (and none of them before it: the vmcnt count below rests on the order)
+    __builtin_amdgcn_sched_barrier(0);   // (and no store or load before it: the vmcnt counts below rest on the order)
     float sc[RPW], rc[RPW];
 #pragma unroll
     for (int rho = 0; rho < RPW; ++rho) {

@@ -6,6 +6,7 @@ vector-register lanes (v_writelane / v_readlane: the persistent 256 x 256 GEMM k
 across the tile loop) touch no memory and are allowed as long as the kernel uses no scratch at all."""
 import csv
 import os
+import re
 
 import pytest
 
@@ -38,3 +39,15 @@ def test_scalar_spills_stay_in_vector_lanes():
     rows = [r for r in _rows() if int(r["sgpr_spill"] or 0)]
     assert all(int(r["scratch"] or 0) == 0 for r in rows)
     assert all("gemm_dma_kernel<4, 2, 4, 5, 1," in r["kernel"] for r in rows), [r["kernel"][:80] for r in rows]
+
+
+def test_wide_kernel_fences_every_dma():
+    """The wide-row kernel's vmcnt waits count the vector-memory instructions issued after each L1^T slab's LDS-DMA, so a
+    scheduling fence follows every slab's DMA: the compiler may otherwise mix two slabs' (they fill separate arrays) or
+    move a store across one, and a slab would be read before it has landed."""
+    with open(os.path.join(ROOT, "pyraquant_amd", "csrc", "pq_quant.hip")) as f:
+        src = re.sub(r"//[^\n]*", "", f.read())
+    body = src[src.index("void quant_lowrank_wide_kernel("):src.index("void lowrank_partial_kernel(")]
+    issues = re.findall(r"dma_l\([^)]*\);\s*(\w+\([^)]*\))", body)
+    assert len(issues) == 3 and body.count("dma_l(") == 3, issues
+    assert all(i == "__builtin_amdgcn_sched_barrier(0)" for i in issues), issues
