@@ -4,8 +4,9 @@
 //
 // One call takes the place of the checks, the two allocations and the twenty-argument foreign call of
 // Int8Linear._forward_direct: an eager layer of few rows (one launch) costs the host 5.0 us, 14.2 before (two launches,
-// 5.5 us, and the rest Python and the foreign call). It looks its tensors up and checks them on every call; nothing is
-// kept between calls. It takes layers without a low-rank branch, whose tensors and x are plain torch tensors in the state
+// 5.5 us, and the rest Python and the foreign call). It looks its tensors up and checks them on every call, and holds them
+// until the launch (the module may be given others meanwhile: by another thread while the GIL is released, or by a dispatch
+// mode's Python during an allocation); nothing is kept between calls. It takes layers without a low-rank branch, whose tensors and x are plain torch tensors in the state
 // the kernels read; for everything else it returns None and the Python paths decide, as they do without it. Results,
 // allocations (torch's caching allocator, on the current stream) and refusals are those of the Python path.
 #include <Python.h>
@@ -80,6 +81,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (PyErr_Occurred()) return nullptr;
     Py_RETURN_NONE;
   }
+  const at::Tensor weight = THPVariable_Unpack(wo), scale = THPVariable_Unpack(so);
+  const at::Tensor bias = bo && bo != Py_None ? THPVariable_Unpack(bo) : at::Tensor();
   const at::Tensor x2 = x.dim() == 2 ? x : x.reshape({-1, K});
   const int64_t M = x2.size(0), ldx = x2.stride(0);
   const void* const xp = x2.const_data_ptr();
@@ -89,10 +92,9 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   int st = PQ_OK;
   if (M > 0) {
     const int32_t code = bf16 ? PQ_BF16 : PQ_F16;
-    const int8_t* const w = static_cast<const int8_t*>(THPVariable_Unpack(wo).const_data_ptr());
-    const float* const s = static_cast<const float*>(THPVariable_Unpack(so).const_data_ptr());
-    const float* const b =
-        bo && bo != Py_None ? static_cast<const float*>(THPVariable_Unpack(bo).const_data_ptr()) : nullptr;
+    const int8_t* const w = static_cast<const int8_t*>(weight.const_data_ptr());
+    const float* const s = static_cast<const float*>(scale.const_data_ptr());
+    const float* const b = bias.defined() ? static_cast<const float*>(bias.const_data_ptr()) : nullptr;
     void* const yp = y.data_ptr();
     const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
     bool taken = false;

@@ -1,5 +1,6 @@
 """The native layer call (_direct.so) that Int8Linear.forward tries first: bit-identical to the Python paths, and it
 steps aside (None) or refuses exactly where they decide."""
+import gc
 import threading
 
 import pytest
@@ -123,3 +124,38 @@ def test_native_call_streams_threads_and_graphs(cuda):
             eager = q(x)
             torch.cuda.synchronize()
             assert torch.equal(y, ref) and torch.equal(eager, ref)
+
+
+@pytest.mark.parametrize("M,swap_at", [(20, 0), (1500, 0), (1500, 1)])   # one kernel; two, and a workspace
+def test_native_call_holds_its_tensors(cuda, M, swap_at):
+    """A module given other buffers during the call (here by a dispatch mode, at one of the call's own allocations) does
+    not take the old ones away from it: their memory is still theirs when the kernels are launched."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    q = _layer(cuda)
+    names = ("weight_packed", "w_scale", "bias")
+    x = torch.randn(M, 1280, device=cuda).bfloat16()
+    ref = q(x)
+    torch.cuda.synchronize()
+    new = {n: torch.zeros_like(q._buffers[n]) for n in names}
+    poison = []
+
+    class Swap(TorchDispatchMode):
+        calls = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            if func is torch.ops.aten.empty.memory_format:
+                if self.calls == swap_at:
+                    before = torch.cuda.memory_allocated()
+                    q._buffers.update(new)
+                    assert torch.cuda.memory_allocated() == before, "the call's tensors have been freed"
+                    poison.extend(torch.full_like(t, 7) for t in new.values())
+                self.calls += 1
+            return out
+
+    gc.collect()   # (other tests' cycles would count as freed here)
+    with Swap() as mode:
+        y = q(x)
+    assert mode.calls == (1 if M < 100 else 2) and len(poison) == 3
+    assert torch.equal(y, ref) and torch.equal(q(x), torch.zeros_like(ref))
