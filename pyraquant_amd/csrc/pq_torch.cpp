@@ -30,7 +30,8 @@ const char* const kNameText[kNames] = {"weight_packed", "w_scale",     "w_scale_
                                        "lr_A",          "group_size",  "in_features", "out_features"};
 PyObject* g_name[kNames];
 
-// An attribute as nn.Module resolves it: the instance's own dict first, then the registered buffers (borrowed).
+// An attribute as nn.Module resolves it: the instance's own dict first, then the registered buffers (borrowed). A name in
+// neither is not None: it may be a parameter or a property, and Python decides.
 PyObject* attribute(PyObject* inst, PyObject* buffers, Name n) {
   PyObject* v = PyDict_GetItemWithError(inst, g_name[n]);
   if (!v && !PyErr_Occurred()) v = PyDict_GetItemWithError(buffers, g_name[n]);
@@ -62,7 +63,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const at::Tensor& x = THPVariable_Unpack(args[2]);
   PyObject* const lr = attribute(inst, buffers, kLrA);
   int64_t K, N, group;
-  if ((lr && lr != Py_None) || !integer(attribute(inst, buffers, kIn), K) || !integer(attribute(inst, buffers, kOut), N) ||
+  if (lr != Py_None || !integer(attribute(inst, buffers, kIn), K) || !integer(attribute(inst, buffers, kOut), N) ||
       !integer(attribute(inst, buffers, kGroup), group)) {
     if (PyErr_Occurred()) return nullptr;
     Py_RETURN_NONE;
@@ -77,12 +78,12 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   PyObject* const so = attribute(inst, buffers, group ? kScaleGroups : kScale);
   PyObject* const bo = attribute(inst, buffers, kBias);
   if (!plain(wo, at::kChar, (N + 15) / 16 * 16 * K, dev) || !plain(so, at::kFloat, group ? N * K / 32 : N, dev) ||
-      (bo && bo != Py_None && !plain(bo, at::kFloat, N, dev))) {
+      (bo != Py_None && !plain(bo, at::kFloat, N, dev))) {
     if (PyErr_Occurred()) return nullptr;
     Py_RETURN_NONE;
   }
   const at::Tensor weight = THPVariable_Unpack(wo), scale = THPVariable_Unpack(so);
-  const at::Tensor bias = bo && bo != Py_None ? THPVariable_Unpack(bo) : at::Tensor();
+  const at::Tensor bias = bo != Py_None ? THPVariable_Unpack(bo) : at::Tensor();
   const at::Tensor x2 = x.dim() == 2 ? x : x.reshape({-1, K});
   const int64_t M = x2.size(0), ldx = x2.stride(0);
   const void* const xp = x2.const_data_ptr();

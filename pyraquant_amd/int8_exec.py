@@ -549,13 +549,14 @@ class Int8Linear(nn.Module):
         return self.lr_Bt
 
     # The tensors the direct call reads through raw pointers, looked up as nn.Module resolves attributes (instance
-    # dict first, then the registered buffers) without its __getattr__: a replaced, moved or re-registered one
-    # changes this tuple's identities and rebuilds the call's plan.
+    # dict first, then the registered buffers; its __getattr__ only for a name in neither, one made a parameter): a
+    # replaced, moved or re-registered one changes this tuple's identities and rebuilds the call's plan.
     _DIRECT_SOURCES = ("weight_packed", "w_scale", "w_scale_gn", "bias", "lr_A", "lr_At", "lr_Bt")
 
     def _direct_sources(self) -> tuple:
         d, b = self.__dict__, self._buffers
-        return tuple(d[n] if n in d else b.get(n) for n in self._DIRECT_SOURCES) + (self._lr_frag(), self.group_size)
+        return (tuple(d[n] if n in d else b[n] if n in b else getattr(self, n) for n in self._DIRECT_SOURCES)
+                + (self._lr_frag(), self.group_size))
 
     def _direct_plan(self, dt: torch.dtype, src: tuple):
         """The part of the direct call that depends on the module alone, for input dtype dt: (source ids, the

@@ -159,3 +159,21 @@ def test_native_call_holds_its_tensors(cuda, M, swap_at):
         y = q(x)
     assert mode.calls == (1 if M < 100 else 2) and len(poison) == 3
     assert torch.equal(y, ref) and torch.equal(q(x), torch.zeros_like(ref))
+
+
+@pytest.mark.parametrize("rank", [0, 32])
+def test_buffers_made_parameters(cuda, rank):
+    """A bias, or a low-rank factor, that the user has made an nn.Parameter is no longer a buffer and still counts."""
+    from pyraquant_amd import _lib
+
+    q = _layer(cuda, rank=rank)
+    x = torch.randn(64, 1280, device=cuda).bfloat16()
+    y = q(x)
+    q.bias = torch.nn.Parameter(q.bias + 1)
+    assert _lib.load_direct()(q.__dict__, q._buffers, x) is None
+    assert torch.equal(q(x), _general(q, x)) and not torch.equal(q(x), y)
+    if rank:
+        p = _layer(cuda, rank=rank)
+        p.lr_A = torch.nn.Parameter(p.lr_A)
+        assert _lib.load_direct()(p.__dict__, p._buffers, x) is None
+        assert torch.equal(p(x), y) and torch.equal(_general(p, x), y)
