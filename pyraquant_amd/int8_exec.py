@@ -630,11 +630,13 @@ class Int8Linear(nn.Module):
         if accumulate:
             assert out is not None, "accumulate=True adds into out="
         if row_idx is None and out is None and out_row_idx is None and DIRECT_CALLS:
-            y = (_direct_linear or _load_direct())(self.__dict__, self._buffers, x)   # no low-rank branch: native
-            if y is not None:
-                if type(y) is int:
-                    _lib.check(y, "int8_linear")
-                return y
+            d, b = self.__dict__, self._buffers
+            if d.get("lr_A", d) is None and d.get("weight_packed", b.get("weight_packed")) is not None:
+                y = (_direct_linear or _load_direct())(d, b, x)   # no low-rank branch: native
+                if y is not None:
+                    if type(y) is int:
+                        _lib.check(y, "int8_linear")
+                    return y
             if self.weight_packed is not None:
                 y = self._forward_direct(x)
                 if y is not None:

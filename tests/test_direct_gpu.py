@@ -177,3 +177,23 @@ def test_buffers_made_parameters(cuda, rank):
         p.lr_A = torch.nn.Parameter(p.lr_A)
         assert _lib.load_direct()(p.__dict__, p._buffers, x) is None
         assert torch.equal(p(x), y) and torch.equal(_general(p, x), y)
+
+
+def test_native_call_is_loaded_for_its_own_layers_only(cuda, monkeypatch):
+    """Where _direct.so does not load, layers it cannot take (a low-rank branch, no packed weights) run as ever; one it
+    takes says so."""
+    from pyraquant_amd import _lib
+    from pyraquant_amd import int8_exec as E
+
+    def missing():
+        raise _lib.LibraryMissing("not built")
+
+    monkeypatch.setattr(_lib, "load_direct", missing)
+    monkeypatch.setattr(E, "_direct_linear", None)
+    x = torch.randn(64, 1280, device=cuda).bfloat16()
+    unpacked = _layer(cuda)
+    unpacked.weight_packed = None
+    for q in (_layer(cuda, rank=32), unpacked):
+        assert torch.equal(q(x), _general(q, x))
+    with pytest.raises(_lib.LibraryMissing):
+        _layer(cuda)(x)
