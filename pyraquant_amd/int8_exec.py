@@ -389,11 +389,13 @@ def _convert_weight(w: torch.Tensor, group_size: int, pack: bool):
     """(codes [N, K], scales, codes in the packed K64 layout or None), pq_convert_weight."""
     assert w.dim() == 2 and w.is_cuda, "weight quantization runs on the GPU (move the Linear to the device first)"
     wk = w.detach()
-    if wk.dtype not in _WEIGHT_DTYPES:
+    if wk.dtype not in _WEIGHT_DTYPES or type(wk) is not torch.Tensor:   # (a subclass says itself what its values are)
         wk = wk.float()
-    if wk.stride(1) != 1:
-        wk = wk.contiguous()
+    wk = wk.resolve_neg()
     N, K = wk.shape
+    # the kernels read a 16-bit weight in place: dense, where its elements or its rows are not (an expanded row, windows)
+    if wk.stride(1) != 1 or (wk.dtype != torch.float32 and wk.stride(0) < K):
+        wk = wk.contiguous()
     if group_size:
         assert K % group_size == 0, (K, group_size)
     q = torch.empty((N, K), dtype=torch.int8, device=w.device)

@@ -281,3 +281,31 @@ def test_convert_weight_one_pass(cuda, dtype, K, group):
     q, s = E.quantize_weight(finite.to(cuda), group)
     qo, so = O.quant_weight(finite.float().numpy(), group)
     assert (q.cpu().numpy() == qo).all() and (s.cpu().numpy() == so).all()
+
+
+@pytest.mark.parametrize("group", [0, 32])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_convert_weight_views(cuda, dtype, group):
+    """Weights that are not dense matrices give the codes and scales of the dense one: rows that overlap (16-bit ones,
+    which are read in place where they can be), a column slice, a transpose, an expanded column, a negated view, and a
+    tensor subclass with values of its own."""
+    from pyraquant_amd import int8_exec as E
+
+    class Doubled(torch.Tensor):
+        def float(self):
+            return self.as_subclass(torch.Tensor).float() * 2
+
+    N, K = 64, 128
+    base = (torch.randn(N * 2 * K, generator=torch.Generator().manual_seed(3)) * 0.02).to(dtype).to(cuda)
+    views = {"slice": base.view(N, 2 * K)[:, :K], "transpose": base[:N * K].view(K, N).t(),
+             "expanded column": base[:N, None].expand(N, K), "negated": torch._neg_view(base[:N * K].view(N, K))}
+    if dtype != torch.float32:
+        views.update({"expanded row": base[:K].expand(N, K), "windows": base.as_strided((N, K), (8, 1)),
+                      "odd windows": base.as_strided((N, K), (3, 1))})
+    cases = {n: (v, v.cpu().clone().to(cuda)) for n, v in views.items()}
+    dense = base[:N * K].view(N, K)
+    cases["subclass"] = (dense.as_subclass(Doubled), dense.float() * 2)
+    for name, (view, ref) in cases.items():
+        q, s, qp = E._convert_weight(view, group, True)
+        q0, s0, qp0 = E._convert_weight(ref.resolve_neg().contiguous(), group, True)
+        assert torch.equal(q, q0) and torch.equal(s, s0) and torch.equal(qp, qp0), name
