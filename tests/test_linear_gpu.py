@@ -534,3 +534,34 @@ def test_int8linear_few_rows_one_kernel(cuda, M, K, N, dtype, bias, pad):
             exact = exact + lin.bias.double()
         lim = exact.abs() * 2.0 ** (-8 if dtype == torch.bfloat16 else -10) + 1e-6
         assert bool(((y.double() - exact).abs() <= lim).all())
+
+
+@pytest.mark.parametrize("M,K,N,shift", [(100, 1280, 1280, 0), (16, 64, 64, 0), (100, 640, 640, 640), (100, 640, 640, -640 * 50),
+                                         (300, 1280, 1280, 0)])
+def test_layer_over_its_input(cuda, M, K, N, shift):
+    """pq_int8_linear and pq_int8_linear_noalloc with y on x, or `shift` elements after it: all of x is read before y is
+    written, also for the sizes that run as one kernel elsewhere."""
+    import ctypes
+
+    from pyraquant_amd import _lib
+    from pyraquant_amd import int8_exec as E
+    from pyraquant_amd.workloads import make_linear, make_x
+
+    L = _lib.load()
+    q = E.Int8Linear(make_linear(K, N, 0, True), device=cuda)
+    xv = make_x(M, K, torch.bfloat16, seed=M + K, device=cuda)
+    ref = q(xv)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ws = torch.empty(L.pq_int8_linear_workspace_size(M, K, 0), dtype=torch.uint8, device=cuda)
+    for noalloc in (False, True):
+        buf = torch.zeros(3 * M * K, dtype=torch.bfloat16, device=cuda)
+        x = buf[M * K:2 * M * K].view(M, K)
+        y = buf[M * K + shift:2 * M * K + shift].view(M, N)
+        x.copy_(xv)
+        args = [p(x), _lib.PQ_BF16, M, K, K, p(q.weight_packed), p(q.w_scale), 0, p(q.bias), None, None, 0, None, 0, p(y), N, N]
+        if noalloc:
+            _lib.check(L.pq_int8_linear_noalloc(*args, stream), "pq_int8_linear_noalloc")
+        else:
+            _lib.check(L.pq_int8_linear(*args, p(ws), ws.numel(), stream), "pq_int8_linear")
+        assert torch.equal(y, ref)
