@@ -1515,8 +1515,8 @@ int pq::quant_rows_lowrank_z(const void* x, int32_t x_dtype, int64_t M, int64_t 
   return set_error(PQ_ESHAPE, "pq_quant_rows_lowrank: unsupported shape");
 }
 
-// The layer as one kernel, or `taken` false where its shape, size or alignment is the two kernels'. y over x is theirs as
-// well: they have read all of x before they write y, the one kernel has not.
+// The layer as one kernel, or `taken` false where its shape, size or alignment is the two kernels' (or not theirs either:
+// they refuse it). y over x is theirs as well: they have read all of x before they write y, the one kernel has not.
 int pq::linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,
                      const float* s_w, const float* bias, void* y, int64_t ldy, int64_t N, bool& taken,
                      hipStream_t stream) {
@@ -1524,7 +1524,7 @@ int pq::linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64
   taken = blocks <= kSmallBlocks && K <= kSmallMaxK && K % 64 == 0 && N % kSmallCols == 0 && ldx >= K && ldx % 8 == 0 && ldy >= N &&
           ldy % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_packed % 16 == 0 && (uintptr_t)s_w % 16 == 0 &&
           (uintptr_t)bias % 16 == 0 && (uintptr_t)y % 8 == 0 && x && w_packed && s_w && y &&
-          (x_dtype == PQ_BF16 || x_dtype == PQ_F16) && M > 0;
+          (x_dtype == PQ_BF16 || x_dtype == PQ_F16) && M > 0 && ldy <= 0x7fffffffLL;
   if (taken) {
     const uintptr_t x0 = (uintptr_t)x, x1 = x0 + 2 * ((M - 1) * ldx + K), y0 = (uintptr_t)y, y1 = y0 + 2 * ((M - 1) * ldy + N);
     taken = x1 <= y0 || y1 <= x0;

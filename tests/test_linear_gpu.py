@@ -565,3 +565,29 @@ def test_layer_over_its_input(cuda, M, K, N, shift):
         else:
             _lib.check(L.pq_int8_linear(*args, p(ws), ws.numel(), stream), "pq_int8_linear")
         assert torch.equal(y, ref)
+
+
+def test_small_layer_refusals(cuda):
+    """What the two kernels refuse is refused at the sizes that run as one kernel too."""
+    import ctypes
+
+    from pyraquant_amd import _lib
+    from pyraquant_amd import int8_exec as E
+    from pyraquant_amd.workloads import make_linear, make_x
+
+    L = _lib.load()
+    q = E.Int8Linear(make_linear(64, 64, 0, False), device=cuda)
+    x, y = make_x(1, 64, torch.bfloat16, seed=1, device=cuda), torch.zeros(1, 64, dtype=torch.bfloat16, device=cuda)
+    p = lambda t, off=0: ctypes.c_void_p(t.data_ptr() + off)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ws = torch.empty(L.pq_int8_linear_workspace_size(1, 64, 0), dtype=torch.uint8, device=cuda)
+
+    def call(dt=_lib.PQ_BF16, ldx=64, ldy=64, out=None, scale=None, bytes=None):
+        return L.pq_int8_linear(p(x), dt, 1, 64, ldx, p(q.weight_packed), scale or p(q.w_scale), 0, None, None, None, 0, None, 0,
+                                out or p(y), ldy, 64, p(ws), ws.numel() if bytes is None else bytes, stream)
+
+    assert call() == _lib.PQ_OK
+    for st, kw in ((_lib.PQ_ESHAPE, dict(ldy=2 ** 31)), (_lib.PQ_EALIGN, dict(ldy=60)), (_lib.PQ_EALIGN, dict(ldy=66)),
+                   (_lib.PQ_EALIGN, dict(out=p(y, 2))), (_lib.PQ_EALIGN, dict(scale=p(q.w_scale, 4))),
+                   (_lib.PQ_ESHAPE, dict(ldx=56)), (_lib.PQ_EDTYPE, dict(dt=_lib.PQ_F32)), (_lib.PQ_ESHAPE, dict(bytes=64))):
+        assert call(**kw) == st, (st, kw)
