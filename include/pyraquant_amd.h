@@ -232,7 +232,7 @@ int64_t pq_int8_linear_workspace_size(int64_t M, int64_t K, int64_t R);
  * x's dtype (R a multiple of 32 up to 128, Re in {16, 32, 64} and Re <= R: the first Re columns of t enter the
  * epilogue), or NULL with R = Re = 0; l1f NULL or l1t in fragment order (as pq_quant_rows_lowrank); y [M, N] in
  * x's dtype with row stride ldy, which may overlap x. Same results as the two calls. Small layers (R == 0, group 0, K <= 4096
- * and at most 320 blocks of 16 rows x 64 outputs) run as one kernel and leave the workspace as it is. The workspace also holds the GEMM's scheduling
+ * and at most 320 blocks of 16 rows x 64 outputs, past K = 2048 at most one per compute unit) run as one kernel and leave the workspace as it is. The workspace also holds the GEMM's scheduling
  * buffer (pq_int8_gemm's sched), which the quantizer kernel zeroes, so a large layer claims its blocks even when
  * replayed from a graph; calls that may overlap need workspaces of their own.
  * Replaces the body of `Int8Linear.forward` (deploy/int8_exec.py:382-393): one C call per layer.

@@ -30,6 +30,10 @@ int quant_rows_lowrank_z(const void* x, int32_t x_dtype, int64_t M, int64_t K, i
                          const int32_t* row_idx, const void* l1t, const void* l1f, int64_t R, int8_t* qp, float* s,
                          void* t, int64_t ldt, int32_t* zero9, hipStream_t stream);
 
+// Compute units of the stream's device, rounded down to a multiple of the 8 XCDs (a persistent grid keeps workgroup
+// b on XCD b % 8); 0 if unknown (pq_gemm.hip).
+int persistent_workgroups(hipStream_t stream);
+
 // The whole layer as one kernel where it has few rows (pq_quant.hip): per-channel weights, no low-rank branch. `taken`
 // says whether it was launched.
 int linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,

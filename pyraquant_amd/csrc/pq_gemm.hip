@@ -1123,8 +1123,8 @@ constexpr int ring_stages() {
   return ns < 8 ? ns : 8;
 }
 
-// Compute units of the stream's device, rounded down to a multiple of the 8 XCDs (a persistent grid keeps workgroup
-// b on XCD b % 8); 0 if unknown.
+}  // namespace
+
 int persistent_workgroups(hipStream_t stream) {
   static std::atomic<int> cached[64];
   int dev = -1;
@@ -1145,6 +1145,8 @@ int persistent_workgroups(hipStream_t stream) {
   if (dev < 64) cached[dev].store(cus, std::memory_order_relaxed);
   return cus;
 }
+
+namespace {
 
 template <int TI, int TJ, int WMW, int OCC, bool PACKED, int MODE, int LRS, int LRDT, int ODT, bool ACC = false>
 int launch_dma(GemmArgs& a, hipStream_t stream) {

@@ -1176,7 +1176,13 @@ constexpr int kSmallMaxK = 4096;   // 64 KB of codes
 // 154 x 2048 x 1280 (200 workgroups) 7.5 us against 3.7 + 5.9, 77 x 4096 x 1280 (100) 10.1 against 4.4 + 7.6, 512 x 640 x
 // 640 (320) 7.9 against 3.2 + 4.9, 256 x 1280 x 1280 (320) 8.9 against 3.7 + 5.8; then the repeated quantizer work loses:
 // 640 x 2048 x 640 (400) 11.4 against 4.3 + 6.3, 512 x 1280 x 1280 (640) 13.5 against 3.8 + 7.2.
+// Past K = 2048 a workgroup's LDS (64 KB of codes and 32 KB of partial sums) leaves room for one per CU, and those past
+// the CUs take a second round. One kernel and two, replayed from a graph over eight layers: at K = 2112, 128 x 2048 (256
+// workgroups) 7.4 and 9.9 us, 96 x 3072 (288) 12.8 and 10.0; at K = 3072 the same rows 8.6 and 10.8, 15.1 and 10.8; at K =
+// 4096, 256 x 1024 (256) 9.4 and 12.9, 77 x 4096 (320) 16.9 and 12.2, 16 x 20480 (320) 26.1 and 24.0. At K = 2048 two fit:
+// 96 x 3072 (288) 8.6 and 9.4, 77 x 4096 (320) 8.6 and 9.3.
 constexpr int64_t kSmallBlocks = 320;
+constexpr int64_t kSmallTwoPerCuK = 2048;
 
 template <int DT, int CH>   // rows of at most 512 CH elements
 __global__ __launch_bounds__(64 * kSmallWaves) void linear_small_kernel(
@@ -1521,7 +1527,12 @@ int pq::linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64
                      const float* s_w, const float* bias, void* y, int64_t ldy, int64_t N, bool& taken,
                      hipStream_t stream) {
   const int64_t blocks = (M + kSmallRows - 1) / kSmallRows * (N / kSmallCols);
-  taken = blocks <= kSmallBlocks && K <= kSmallMaxK && K % 64 == 0 && N % kSmallCols == 0 && ldx >= K && ldx % 8 == 0 && ldy >= N &&
+  int64_t most = kSmallBlocks;
+  if (K > kSmallTwoPerCuK) {
+    const int cus = persistent_workgroups(stream);
+    most = std::min<int64_t>(most, cus > 0 ? cus : 256);
+  }
+  taken = blocks <= most && K <= kSmallMaxK && K % 64 == 0 && N % kSmallCols == 0 && ldx >= K && ldx % 8 == 0 && ldy >= N &&
           ldy % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_packed % 16 == 0 && (uintptr_t)s_w % 16 == 0 &&
           (uintptr_t)bias % 16 == 0 && (uintptr_t)y % 8 == 0 && x && w_packed && s_w && y &&
           (x_dtype == PQ_BF16 || x_dtype == PQ_F16) && M > 0 && ldy <= 0x7fffffffLL;

@@ -591,3 +591,31 @@ def test_small_layer_refusals(cuda):
                    (_lib.PQ_EALIGN, dict(out=p(y, 2))), (_lib.PQ_EALIGN, dict(scale=p(q.w_scale, 4))),
                    (_lib.PQ_ESHAPE, dict(ldx=56)), (_lib.PQ_EDTYPE, dict(dt=_lib.PQ_F32)), (_lib.PQ_ESHAPE, dict(bytes=64))):
         assert call(**kw) == st, (st, kw)
+
+
+@pytest.mark.parametrize("K,per_cu", [(1024, 0), (2048, 0), (2112, 1), (4096, 1)])
+def test_one_kernel_where_its_blocks_fit(cuda, K, per_cu):
+    """The layer runs as one kernel (which leaves the workspace as it is) up to 320 blocks of 16 rows x 64 outputs, and past
+    K = 2048, where one block fits a compute unit, up to the compute units; both sides of the line, the same bits."""
+    import ctypes
+
+    from pyraquant_amd import _lib
+    from pyraquant_amd import int8_exec as E
+    from pyraquant_amd.workloads import make_linear, make_x
+
+    L = _lib.load()
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count // 8 * 8
+    most = min(320, cus) if per_cu else 320
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for blocks in (most, most + 1):
+        M, N = 16, blocks * 64
+        q = E.Int8Linear(make_linear(K, N, 0, True), device=cuda)
+        x = make_x(M, K, torch.bfloat16, seed=K, device=cuda)
+        ws = torch.full((L.pq_int8_linear_workspace_size(M, K, 0),), 0x5a, dtype=torch.uint8, device=cuda)
+        y = torch.empty(M, N, dtype=torch.bfloat16, device=cuda)
+        _lib.check(L.pq_int8_linear(p(x), _lib.PQ_BF16, M, K, K, p(q.weight_packed), p(q.w_scale), 0, p(q.bias), None, None, 0,
+                                    None, 0, p(y), N, N, p(ws), ws.numel(), stream), "pq_int8_linear")
+        assert bool((ws == 0x5a).all()) == (blocks <= most), blocks
+        xq, sx = E.quant_rows_packed(x)
+        assert torch.equal(y, E.int8_gemm_packed(xq, sx, q.weight_packed, q.w_scale, q.bias, M, N, K, x.dtype))
