@@ -34,8 +34,9 @@ int quant_rows_lowrank_z(const void* x, int32_t x_dtype, int64_t M, int64_t K, i
 // b on XCD b % 8); 0 if unknown (pq_gemm.hip).
 int persistent_workgroups(hipStream_t stream);
 
-// The whole layer as one kernel where it has few rows (pq_quant.hip): per-channel weights, no low-rank branch. `taken`
-// says whether it was launched.
+// The whole layer as one kernel where it has few rows (pq_quant.hip): per-channel weights, no low-rank branch.
+// linear_small_size: whether it is of such a size. linear_small: `taken` says whether it was launched.
+bool linear_small_size(int64_t M, int64_t K, int64_t N, hipStream_t stream);
 int linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,
                  const float* s_w, const float* bias, void* y, int64_t ldy, int64_t N, bool& taken, hipStream_t stream);
 

@@ -1521,19 +1521,22 @@ int pq::quant_rows_lowrank_z(const void* x, int32_t x_dtype, int64_t M, int64_t 
   return set_error(PQ_ESHAPE, "pq_quant_rows_lowrank: unsupported shape");
 }
 
-// The layer as one kernel, or `taken` false where its shape, size or alignment is the two kernels' (or not theirs either:
-// they refuse it). y over x is theirs as well: they have read all of x before they write y, the one kernel has not.
-int pq::linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,
-                     const float* s_w, const float* bias, void* y, int64_t ldy, int64_t N, bool& taken,
-                     hipStream_t stream) {
+bool pq::linear_small_size(int64_t M, int64_t K, int64_t N, hipStream_t stream) {
   const int64_t blocks = (M + kSmallRows - 1) / kSmallRows * (N / kSmallCols);
   int64_t most = kSmallBlocks;
   if (K > kSmallTwoPerCuK) {
     const int cus = persistent_workgroups(stream);
     most = std::min<int64_t>(most, cus > 0 ? cus : 256);
   }
-  taken = blocks <= most && K <= kSmallMaxK && K % 64 == 0 && N % kSmallCols == 0 && ldx >= K && ldx % 8 == 0 && ldy >= N &&
-          ldy % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_packed % 16 == 0 && (uintptr_t)s_w % 16 == 0 &&
+  return blocks <= most && K <= kSmallMaxK && K % 64 == 0 && N % kSmallCols == 0;
+}
+
+// The layer as one kernel, or `taken` false where its shape, size or alignment is the two kernels' (or not theirs either:
+// they refuse it). y over x is theirs as well: they have read all of x before they write y, the one kernel has not.
+int pq::linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* w_packed,
+                     const float* s_w, const float* bias, void* y, int64_t ldy, int64_t N, bool& taken,
+                     hipStream_t stream) {
+  taken = linear_small_size(M, K, N, stream) && ldx >= K && ldx % 8 == 0 && ldy >= N && ldy % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_packed % 16 == 0 && (uintptr_t)s_w % 16 == 0 &&
           (uintptr_t)bias % 16 == 0 && (uintptr_t)y % 8 == 0 && x && w_packed && s_w && y &&
           (x_dtype == PQ_BF16 || x_dtype == PQ_F16) && M > 0 && ldy <= 0x7fffffffLL;
   if (taken) {
@@ -1541,7 +1544,7 @@ int pq::linear_small(const void* x, int32_t x_dtype, int64_t M, int64_t K, int64
     taken = x1 <= y0 || y1 <= x0;
   }
   if (!taken) return PQ_OK;
-  const dim3 grid((unsigned)blocks), block(64 * kSmallWaves);
+  const dim3 grid((unsigned)((M + kSmallRows - 1) / kSmallRows * (N / kSmallCols))), block(64 * kSmallWaves);
   const uint16_t* xp = static_cast<const uint16_t*>(x);
   uint16_t* yp = static_cast<uint16_t*>(y);
 #define PQ_SMALL(D, C)                                                                                                  \

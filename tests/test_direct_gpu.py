@@ -197,3 +197,30 @@ def test_native_call_is_loaded_for_its_own_layers_only(cuda, monkeypatch):
         assert torch.equal(q(x), _general(q, x))
     with pytest.raises(_lib.LibraryMissing):
         _layer(cuda)(x)
+
+
+def test_native_call_allocates_as_the_python_path(cuda):
+    """The workspace before the output, so that consecutive calls take the same workspace and outputs of their own; a
+    layer of few rows allocates its output alone."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Sizes(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            if func is torch.ops.aten.empty.memory_format:
+                self.seen.append((out.dtype, out.numel()))
+            return out
+
+    for group, M in ((0, 20), (0, 1500), (32, 20), (32, 1500)):
+        q = _layer(cuda, group=group)
+        x = torch.randn(M, 1280, device=cuda).bfloat16()
+        with Sizes() as native:
+            q(x)
+        with Sizes() as python:
+            q._forward_direct(x)
+        assert [d for d, _ in python.seen] == [torch.uint8, torch.bfloat16]
+        assert native.seen == (python.seen[1:] if group == 0 and M < 100 else python.seen)
