@@ -40,6 +40,7 @@
 // workgroup per CU, which claims its XCD's tiles (then the other XCDs') through a scheduling buffer the caller owns
 // (or, without one, takes a fixed share of them).
 #include "pq_common.h"
+#include "pq_tiles.h"
 
 #include <atomic>
 #include <type_traits>
@@ -919,11 +920,9 @@ void gemm_dma_kernel(const GemmArgs p) {
   // the buffer it steps through its own list (a fixed share per workgroup).
   //
   // Tiles past a list's last whole round (a tile for every workgroup of the XCD) are handed out as four 128 x 128 quarters
-  // where the quarters are no more than the workgroups: a quarter takes about a third of a tile's time, so they end the
-  // product that much earlier (launch_dma sets whole_lo / whole_hi). Measured, start and now: M = 4352, K = 3072, N =
-  // 12288 (3.19 rounds) 163.7 and 158.7 us, 16640 x 3072 x 3072 (3.05) 171.4 and 157.6, 16640 x 12288 x 3072 538.8 and
-  // 495.5; where other XCDs' claims already cover the short round (65792 x 3072 x 3072, 12.05 rounds) the same. Two
-  // rounds of quarters lose: 4352 x 3072 x 9216 (2.39 rounds) 122.3 whole, 132.6 in quarters.
+  // where those end the product earlier (whole_tiles sets whole_lo / whole_hi, and says where that is). Whole and in
+  // quarters: M = 4352, K = 3072, N = 12288 (3.19 rounds) 163.7 and 158.7 us, 16640 x 3072 x 3072 (3.05) 171.4 and 157.6,
+  // 16640 x 12288 x 3072 538.8 and 495.5.
   const int wgx = ((int)gridDim.x + 7) >> 3;   // workgroups per XCD (a grid smaller than the tiles is a multiple of 8)
   const int x0 = blockIdx.x & 7;
   auto xcd_cnt = [&](int x) { return (nbt >> 3) + (x < (nbt & 7) ? 1 : 0); };
@@ -1162,9 +1161,9 @@ int launch_dma(GemmArgs& a, hipStream_t stream) {
     a.whole_lo = lo;
     a.whole_hi = lo + 1;
     if (wg > 0 && grid.x > (unsigned)wg) {
-      const int wgx = wg / 8;
-      a.whole_lo = 4 * (lo % wgx) <= wgx ? lo - lo % wgx : lo;
-      a.whole_hi = 4 * ((lo + 1) % wgx) <= wgx ? lo + 1 - (lo + 1) % wgx : lo + 1;
+      const WholeTiles whole = whole_tiles((int)grid.x, wg / 8, a.K);
+      a.whole_lo = whole.lo;
+      a.whole_hi = whole.hi;
       grid.x = (unsigned)wg;
       a.sched = sched;
     }

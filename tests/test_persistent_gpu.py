@@ -208,18 +208,26 @@ def test_layer_call_fresh_workspace_and_graph(cuda):
         assert torch.equal(y_e, ref), f"eager call beside replay {i}"
 
 
-# 256 x 256 tiles per XCD list over 32 workgroups: 33 and 34 (some lists one tile longer), quarters that hang over the
-# last rows (M % 256 = 56: the lower quarters are empty) and columns (N % 256 = 64), 40 tiles (8 over: the most that go
-# out in quarters) and 41 (whole again)
+# Products of at least 1024 blocks of 128 x 256 (persistent 256 x 256 tiles) by the tiles in an XCD's list, over 32
+# workgroups: 68, with lower and right quarters that lie past the last row (M % 256 = 56) and column (N % 256 = 64); 64
+# and 65, with one K stage; 69 (5 past the round, the most at a short K); 69 and 70, which go out in quarters from
+# K = 2048; 72, the most there are, from K = 4096; 69 and 70 at a short K, and 73: whole
 @pytest.mark.parametrize("sched", [True, False])
-@pytest.mark.parametrize("lr,shape", [(32, (4152, 4096 + 64, 128)), (0, (5120, 4096, 192)), (16, (5248, 4096, 64)),
-                                      (0, (2560, 8192 + 192, 320))])
-def test_last_tiles_in_quarters(cuda, sched, lr, shape):
+@pytest.mark.parametrize("lr,shape,lists,quarters", [
+    (32, (4152, 8000, 128), (68, 68), True), (16, (6882, 4800, 64), (64, 65), True), (0, (5800, 6144 - 64, 192), (69, 69), True),
+    (32, (3840, 9472, 2048), (69, 70), True), (0, (4600, 8192, 4096), (72, 72), True), (0, (3840, 9472, 320), (69, 70), False),
+    (16, (2048, 18688, 192), (73, 73), False)])
+def test_last_tiles_in_quarters(cuda, sched, lr, shape, lists, quarters):
     """Lists that end in a few tiles past a whole round hand those out as 128 x 128 quarters: every tile written, with
     the bits of the one-tile-per-workgroup kernels, with claims and with fixed shares, scattered too."""
     from pyraquant_amd import int8_exec as E
+    from test_tiles_cpu import whole_tiles
 
     M, N, K = shape
+    assert torch.cuda.get_device_properties(cuda).multi_processor_count == 256
+    assert -(-M // 128) * -(-N // 256) >= 1024
+    lengths, whole = whole_tiles(-(-M // 256) * -(-N // 256), K)
+    assert lengths == lists and (whole != lengths) == quarters
     P = _problem(cuda, 5 + lr, lr, shape)
     ref = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
     for r0 in range(0, M, 256):
