@@ -885,7 +885,8 @@ constexpr int tile_lds() {
 // Ring of the quarter tiles (128 x 128 on 8 waves): 8 stages of 16 KB.
 constexpr int kQuarterStages = 8;
 
-template <int TI, int TJ, int WMW, int NS, int OCC, bool PACKED, int MODE, int LRS, int LRDT, int ODT, bool ACC = false>
+template <int TI, int TJ, int WMW, int NS, int OCC, bool PACKED, int MODE, int LRS, int LRDT, int ODT, bool ACC = false,
+          bool QUARTERS = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(128 * WMW, 128 * WMW),
                           amdgpu_waves_per_eu(OCC * WMW / 2, OCC * WMW / 2)))
 void gemm_dma_kernel(const GemmArgs p) {
@@ -922,11 +923,15 @@ void gemm_dma_kernel(const GemmArgs p) {
   // Tiles past a list's last whole round (a tile for every workgroup of the XCD) are handed out as four 128 x 128 quarters
   // where those end the product earlier (whole_tiles sets whole_lo / whole_hi, and says where that is). Whole and in
   // quarters: M = 4352, K = 3072, N = 12288 (3.19 rounds) 163.7 and 158.7 us, 16640 x 3072 x 3072 (3.05) 171.4 and 157.6,
-  // 16640 x 12288 x 3072 538.8 and 495.5.
+  // 16640 x 12288 x 3072 538.8 and 495.5. Products without quarters take a kernel without their loop (QUARTERS): the loop
+  // nearly doubles the scalar registers parked in vector lanes (164 and 335 at rank 32), which the whole tiles pay for:
+  // 0.4-0.6 % at K = 640 and 1280 without a low-rank term, 0.2 % at K = 3072.
   const int wgx = ((int)gridDim.x + 7) >> 3;   // workgroups per XCD (a grid smaller than the tiles is a multiple of 8)
   const int x0 = blockIdx.x & 7;
   auto xcd_cnt = [&](int x) { return (nbt >> 3) + (x < (nbt & 7) ? 1 : 0); };
-  auto xcd_whole = [&](int x) { return x < (nbt & 7) ? p.whole_hi : p.whole_lo; };   // tiles of list x that go out whole
+  auto xcd_whole = [&](int x) {   // tiles of list x that go out whole
+    return !QUARTERS ? xcd_cnt(x) : x < (nbt & 7) ? p.whole_hi : p.whole_lo;
+  };
   auto xcd_entries = [&](int x) { return 4 * xcd_cnt(x) - 3 * xcd_whole(x); };
   // Claims (lane 0 of wave 0). Part 1, issued before the epilogue so that the atomic's round trip overlaps it: the next
   // entry of the own list.
@@ -969,7 +974,7 @@ void gemm_dma_kernel(const GemmArgs p) {
     lds_barrier();   // every wave has read it, and is done with the staging area, before the next tile's DMA
   }
   // Quarters (and a whole tile claimed from another XCD's list meanwhile, as its four quarters).
-  while (vb >= 0) {
+  while (QUARTERS && vb >= 0) {
     const int x = vb & 7, whole = xcd_whole(x), li = vb >> 3, q = li - whole;
     int tm, tn;
     tile_coords<group_m<OCC>()>(((q < 0 ? li : whole + (q >> 2)) << 3) | x, nbt, p.tiles_m, p.tiles_n, tm, tn);
@@ -1162,10 +1167,16 @@ int launch_dma(GemmArgs& a, hipStream_t stream) {
     a.whole_hi = lo + 1;
     if (wg > 0 && grid.x > (unsigned)wg) {
       const WholeTiles whole = whole_tiles((int)grid.x, wg / 8, a.K);
+      const bool quarters = whole.lo < lo || ((grid.x & 7) && whole.hi <= lo);
       a.whole_lo = whole.lo;
       a.whole_hi = whole.hi;
       grid.x = (unsigned)wg;
       a.sched = sched;
+      if (quarters) {
+        hipLaunchKernelGGL((gemm_dma_kernel<TI, TJ, WMW, NS, OCC, PACKED, MODE, LRS, LRDT, ODT, ACC, true>), grid,
+                           dim3(128 * WMW), 0, stream, a);
+        return check_launch("int8_gemm");
+      }
     }
   }
   hipLaunchKernelGGL((gemm_dma_kernel<TI, TJ, WMW, NS, OCC, PACKED, MODE, LRS, LRDT, ODT, ACC>), grid, dim3(128 * WMW), 0,

@@ -41,6 +41,14 @@ def test_scalar_spills_stay_in_vector_lanes():
     assert all("gemm_dma_kernel<4, 2, 4, 5, 1," in r["kernel"] for r in rows), [r["kernel"][:80] for r in rows]
 
 
+def test_products_without_quarters_park_fewer_registers():
+    """The persistent kernel for products whose tiles all go out whole (the last argument false) does not hold the
+    quarters' loop, which nearly doubles the scalar registers parked in vector lanes (up to 181 before there were quarters)."""
+    rows = [r for r in _rows() if "gemm_dma_kernel<4, 2, 4, 5, 1," in r["kernel"] and int(r["sgpr_spill"] or 0)]
+    whole = [r for r in rows if "false>(" in r["kernel"]]
+    assert whole and len(whole) < len(rows) and max(int(r["sgpr_spill"]) for r in whole) <= 181
+
+
 def test_wide_kernel_fences_every_dma():
     """The wide-row kernel's vmcnt waits count the vector-memory instructions issued after each L1^T slab's LDS-DMA, so a
     scheduling fence follows every slab's DMA: the compiler may otherwise mix two slabs' (they fill separate arrays) or
