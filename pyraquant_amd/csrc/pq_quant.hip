@@ -248,16 +248,20 @@ __global__ __launch_bounds__(256) void quant_rows_scalar_kernel(
   const float a = fmaxf(absmax_from_bits<DT>(mx), 1e-8f);
   const float sc = __fdiv_rn(a, 127.0f);
   int8_t* __restrict__ qr = q + m * (int64_t)K;
-  for (int k = lane; k < K; k += 64) {
-    const float f = live ? lo16_to_f32<DT>(xr[k]) : 0.0f;
-    const bool finite = fabsf(f) < __builtin_inff();
-    const int8_t code = finite ? (int8_t)(__float_as_uint(code_exact(f, sc)) & 0xffu) : (int8_t)0;
-    if constexpr (PACKED) {
-      q[k64_offset(m, k, K >> 6)] = code;
-    } else {
-      qr[k] = code;
+  auto sweep = [&](auto finite_row) {
+    for (int k = lane; k < K; k += 64) {
+      const float f = live ? lo16_to_f32<DT>(xr[k]) : 0.0f;
+      const bool finite = decltype(finite_row)::value || fabsf(f) < __builtin_inff();
+      const int8_t code = finite ? (int8_t)(__float_as_uint(code_exact(f, sc)) & 0xffu) : (int8_t)0;
+      if constexpr (PACKED) {
+        q[k64_offset(m, k, K >> 6)] = code;
+      } else {
+        qr[k] = code;
+      }
     }
-  }
+  };
+  if (mx < NanRow<DT>::kInf) sweep(std::true_type{});
+  else sweep(std::false_type{});
   if (lane == 0) s[m] = sc;
 }
 
