@@ -487,7 +487,8 @@ __global__ __launch_bounds__(256) void convert_rows_kernel(const void* __restric
   if (lane == 0) s[n] = sc;
 }
 
-// Rows of any length. G32: groups of 32, whose four lanes share their absmax through two quad permutes, one sweep.
+// Rows of any length. G32: groups of 32, whose four lanes share their absmax through two quad permutes, one sweep; a row's
+// groups are dealt to gridDim.y waves.
 // Otherwise per channel in two sweeps (fp32 rows too long for the registers; the second comes mostly from the L2).
 template <int W, bool G32>
 __global__ __launch_bounds__(256) void convert_sweep_kernel(const void* __restrict__ w, int64_t ldw, int N, int K,
@@ -513,7 +514,7 @@ __global__ __launch_bounds__(256) void convert_sweep_kernel(const void* __restri
     if (lane == 0) s[n] = sc;
   }
 #pragma unroll 4
-  for (int i0 = 0; i0 < nvec; i0 += 64) {   // (every lane stays in the loop: the permutes read whole quads)
+  for (int i0 = 64 * blockIdx.y; i0 < nvec; i0 += 64 * gridDim.y) {   // (every lane stays: the permutes read whole quads)
     const int idx = i0 + lane;
     WChunk<W> c{};
     if (idx < nvec) c = load_wchunk<W>(row, idx);
@@ -1617,7 +1618,11 @@ static int convert_weight(const void* w, int64_t N, int64_t K, int64_t ldw, int6
     const dim3 grid((unsigned)((N + 3) / 4)), block(256);
     const int need = (int)((K / 8 + 63) / 64);
     if (group == 32) {
-      hipLaunchKernelGGL((convert_sweep_kernel<W, true>), grid, block, 0, stream, w, ldw, (int)N, (int)K, q, s, qp);
+      // few rows: K split over up to 4096 waves, 16 per CU. One wave per row and split, 64 x 12288 (fp32) 12.3 and 3.3 us, 640
+      // x 5120 7.4 and 4.4, 1280 x 5120 11.0 and 7.1, 2048 x 12288 30.6 and 28.2; with 3072 rows two waves a row lose
+      // (42.3 and 43.2 at K = 12288).
+      const dim3 split(grid.x, (unsigned)std::max<int64_t>(1, std::min<int64_t>(need, 4096 / N)));
+      hipLaunchKernelGGL((convert_sweep_kernel<W, true>), split, block, 0, stream, w, ldw, (int)N, (int)K, q, s, qp);
       return check_launch("quant_weight");
     }
     // registers: 4 per 16-bit chunk (K <= 15360: 30 chunks), 8 per fp32 chunk (K <= 6144)

@@ -309,3 +309,20 @@ def test_convert_weight_views(cuda, dtype, group):
         q, s, qp = E._convert_weight(view, group, True)
         q0, s0, qp0 = E._convert_weight(ref.resolve_neg().contiguous(), group, True)
         assert torch.equal(q, q0) and torch.equal(s, s0) and torch.equal(qp, qp0), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K", [(1, 544), (16, 2080), (16, 12288), (64, 15392), (1100, 1056), (2048, 1024), (2049, 1024)])
+def test_convert_group32_rows_over_several_waves(cuda, dtype, N, K):
+    """Groups of 32 of few rows, dealt to several waves a row (one from 2049 rows on), with a last step of each row that
+    does not fill a wave: the codes and scales of the element-by-element kernel, and every one of them written."""
+    from pyraquant_amd import int8_exec as E
+
+    w = (torch.randn(N, K, generator=torch.Generator().manual_seed(N)) * 0.02).to(dtype)
+    wide = torch.zeros(N, K + 8, dtype=dtype, device=cuda)
+    wide[:, 1:K + 1] = w.to(cuda)
+    q, s, qp = E._convert_weight(w.to(cuda), 32, K % 64 == 0 and N % 16 == 0)
+    q1, s1 = E.quantize_weight(wide[:, 1:K + 1], 32)
+    assert torch.equal(q, q1) and torch.equal(s, s1)
+    if qp is not None:
+        assert torch.equal(qp, E.pack_k64(q1))
