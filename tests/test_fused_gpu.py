@@ -246,7 +246,8 @@ def test_quant_rows_lowrank_wide_tail(cuda, gather, M, K, dtype):
     """The wide-row rule: rows past the last whole round of one batch per CU take lowrank_partial_kernel and the
     quantizer that finishes t. Codes and scales as the plain quantizer's, bit for bit; t within one 16-bit rounding of
     the float64 product (2^-8 |t| in bf16) plus the fp32 sum's error (K 2^-24 sum |x l1|); gathered rows outside x
-    read as zeros; nothing beside t's own columns is written."""
+    read as zeros; nothing past the rows and beside t's own columns is written."""
+    from pyraquant_amd import _lib
     from pyraquant_amd import int8_exec as E
     from pyraquant_amd.workloads import make_x
 
@@ -260,9 +261,21 @@ def test_quant_rows_lowrank_wide_tail(cuda, gather, M, K, dtype):
         idx[0], idx[M // 2] = rows, -1
         idx = idx.to(cuda)
     xin = x if gather else x[:M]
-    qp, s, t = E.quant_rows_lowrank(xin, l1t, idx)
+    # t with eight columns and three rows more than it needs, codes past the padded rows, scales past M: all kept
+    L, padded, ldt = _lib.load(), E.packed_rows(M) * K, 40
+    qx = torch.full((padded + 16 * K,), 99, dtype=torch.int8, device=cuda)
+    sx = torch.full((M + 16,), -7.0, device=cuda)
+    tx = torch.full((M + 3, ldt), -7.0, dtype=dtype, device=cuda)
+    _lib.check(L.pq_quant_rows_lowrank(_lib.ptr(xin), _lib.dtype_code(dtype), M, K, xin.stride(0), xin.shape[0],
+                                       _lib.ptr(idx), _lib.ptr(l1t), None, 32, _lib.ptr(qx), _lib.ptr(sx), _lib.ptr(tx), ldt,
+                                       _lib.stream_of(cuda)), "quant_rows_lowrank")
+    assert bool((qx[padded:] == 99).all()) and bool((sx[M:] == -7).all())
+    assert bool((tx[M:] == -7).all()) and bool((tx[:, 32:] == -7).all())
+    qp, s, t = qx[:padded], sx[:M], tx[:M, :32]
     qr, sr = E.quant_rows_packed(xin, idx)
     assert torch.equal(qp, qr) and torch.equal(s, sr)
+    qw, sw, tw = E.quant_rows_lowrank(xin, l1t, idx)
+    assert torch.equal(qw, qp) and torch.equal(sw, s) and torch.equal(tw, t)
     xs = x[:M] if idx is None else torch.where(((idx >= 0) & (idx < rows))[:, None], x[idx.clamp(0, rows - 1).long()],
                                                torch.zeros((), dtype=dtype, device=cuda))
     for r0 in range(0, M, 2048):

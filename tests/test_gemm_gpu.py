@@ -16,6 +16,7 @@ import pytest
 import torch
 
 from conftest import MAX_REL, MEAN_REL, bits, dcode, rel_errors
+from dispatch_rules import group32_block
 
 pytestmark = pytest.mark.gpu
 
@@ -185,20 +186,23 @@ def test_gemm_rejects_bad_shapes(cuda):
         E.int8_gemm_fused(a, torch.ones(16, device=cuda), w, torch.ones(96, device=cuda), None, torch.bfloat16)
 
 
-@pytest.mark.parametrize("M,N,K", [
-    # 128 x 64 blocks: up to two 128 x 128 per CU, and above where their last round is the fuller
-    (1, 128, 64), (65, 192, 96 * 2), (2048, 640, 128), (8192, 1280, 64), (10000, 1280, 64),
-    # 128 x 128 blocks at three per CU: 513 blocks, ragged rows (10, 33 and 65 of the last 128, with waves that have
-    # none) and a half-filled last column
-    (65536, 256, 64), (8202, 5120, 192), (16417, 1280, 128), (9025, 1472, 320)])
+@pytest.mark.parametrize("M,N,K,block", [
+    (1, 128, 64, "64 x 32"), (65, 192, 96 * 2, "64 x 32"), (2048, 640, 128, "64 x 32"),
+    # up to two 128 x 128 blocks per CU, and above where their last round is the fuller; a half-filled last column, 65
+    # rows of the last 128
+    (6400, 1280, 128, "128 x 64"), (8192, 1280, 64, "128 x 64"), (10000, 1280, 64, "128 x 64"), (9025, 1472, 320, "128 x 64"),
+    # three per CU: 1024 blocks, ragged rows (10, 33 and 65 of the last 128, with waves that have none), the last with a
+    # half-filled last column too
+    (65536, 256, 64, "128 x 128"), (8202, 5120, 192, "128 x 128"), (16417, 1280, 128, "128 x 128"), (8129, 1472, 320, "128 x 128")])
 @pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.float16, False)])
-def test_group32_blocks(cuda, M, N, K, dtype, bias):
-    """Both group-32 blocks at their limits: each output bit for bit the fp32 chain fma(s_w[g], partial_g, ..) over the
+def test_group32_blocks(cuda, M, N, K, block, dtype, bias):
+    """The group-32 blocks at their limits: each output bit for bit the fp32 chain fma(s_w[g], partial_g, ..) over the
     groups in order, times s_row, plus bias, rounded once (fma evaluated in float64, whose single rounding to fp32 is
     exact here: a 24-bit scale times a 20-bit partial and a 24-bit sum fit 53 bits unless the sum cancels far below its
     terms; those few elements may differ by one rounding of the 16-bit type)."""
     from pyraquant_amd import int8_exec as E
 
+    assert group32_block(M, N) == block
     g = torch.Generator(device=cuda).manual_seed(M + N + K)
     a = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device=cuda)
     w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=cuda)

@@ -8,6 +8,8 @@ import numpy as np
 import pytest
 import torch
 
+from dispatch_rules import channel_block, group32_block
+
 pytestmark = pytest.mark.gpu
 
 PAD = 8
@@ -65,20 +67,23 @@ def test_gather_out_of_range_reads_zero_rows(cuda, dtype, K):
                 assert _bits_equal(tf[~dead], tr[~dead]) and not tf[dead].any()
 
 
-@pytest.mark.parametrize("M,N,K,group,rank,accumulate", [
-    (300, 640, 1280, 0, 32, False),      # 128 x 64 blocks
-    (300, 640, 1280, 0, 32, True),       # the accumulating epilogue (reads the destination row first)
-    (300, 1280, 1280, 32, 0, False),     # group-32
-    (12000, 3072, 1024, 0, 32, False),   # 256 x 256 blocks
-    (12000, 3072, 1024, 0, 0, True),
+@pytest.mark.parametrize("M,N,K,group,rank,accumulate,block", [
+    (300, 640, 1280, 0, 32, False, "split K, 64 x 32"),
+    (300, 640, 1280, 0, 32, True, "split K, 64 x 32"),   # the accumulating epilogue (reads the destination row first)
+    (1700, 640, 1280, 0, 32, False, "128 x 64"),
+    (2048, 3072, 128, 0, 32, True, "128 x 256"),
+    (300, 1280, 1280, 32, 0, False, "64 x 32"),          # group-32
+    (12000, 3072, 1024, 0, 32, False, "256 x 256"),
+    (12000, 3072, 1024, 0, 0, True, "256 x 256"),
 ])
-def test_scatter_out_of_range_rows_not_written(cuda, M, N, K, group, rank, accumulate):
+def test_scatter_out_of_range_rows_not_written(cuda, M, N, K, group, rank, accumulate, block):
     """Int8Linear.forward scattering into a canvas view: rows named outside the canvas are skipped, rows named inside
     it get the layer's output (added to the row with accumulate=True, as torch's 16-bit add rounds it), every other
     row of the canvas and of its parent keeps its bits."""
     from pyraquant_amd import int8_exec as E
     from pyraquant_amd.workloads import make_linear, make_x
 
+    assert (group32_block if group else channel_block)(M, N) == block
     dtype = torch.float16 if group else torch.bfloat16
     q = E.Int8Linear(make_linear(K, N, rank, True, seed=M + N, dtype=dtype), device=cuda, group_size=group)
     x = make_x(M, K, dtype, seed=M, device=cuda)

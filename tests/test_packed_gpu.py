@@ -246,7 +246,7 @@ def test_gemm_one_round_big_tiles(oracle, cuda, M, N, K, lr):
     is exactly one block per CU; the others are ragged in M and N, long in K, or a single 64-wide K stage against
     the ring's five). The int32 accumulators are exact against the oracle on sampled rows, the
     last ragged ones included, row-major and packed. The fused output is bit-identical to the same product computed
-    in 256-row slices, whose few blocks run the 128 x 64 kernel with the same per-element epilogue arithmetic."""
+    in 256-row slices, whose few blocks run the split-K kernel with the same per-element epilogue arithmetic."""
     from pyraquant_amd import int8_exec as E
 
     a, w = _codes(M, N, K, M + N + lr, cuda)

@@ -221,7 +221,7 @@ def test_last_tiles_in_quarters(cuda, sched, lr, shape, lists, quarters):
     """Lists that end in a few tiles past a whole round hand those out as 128 x 128 quarters: every tile written, with
     the bits of the one-tile-per-workgroup kernels, with claims and with fixed shares, scattered too."""
     from pyraquant_amd import int8_exec as E
-    from test_tiles_cpu import whole_tiles
+    from dispatch_rules import whole_tiles
 
     M, N, K = shape
     assert torch.cuda.get_device_properties(cuda).multi_processor_count == 256

@@ -168,14 +168,15 @@ def test_linear_golden_fixture(cuda):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_quant_rows_every_mantissa_pair(oracle, cuda, dtype):
     """Codes come from a branch-free Newton step, whose rounding depends on the row maximum's and the element's
-    mantissas and their exponent difference alone: every maximum (all 128 mantissas in bf16; every fifth of the 1024 in
-    fp16) against every element mantissa at exponent differences 0 .. 9 (below that every code is 0), both signs,
-    against the oracle bit for bit, in the packed and the row-major kernel."""
+    mantissas and their exponent difference alone: every maximum (all 128 mantissas in bf16, all 1024 in fp16) against
+    every element mantissa at exponent differences 0 .. 9 (below that every code is 0), both signs; and the floor's scale
+    (rows with no element above 1e-8, in bf16) against every element that has a code; against the oracle bit for bit,
+    in the packed and the row-major kernel."""
     from pyraquant_amd import int8_exec as E
 
     bf = dtype == torch.bfloat16
-    n, step, base = (128, 1, 0x3F80) if bf else (1024, 5, 0x4C00)
-    maxima = torch.arange(0, n, step) + base
+    n, base = (128, 0x3F80) if bf else (1024, 0x4C00)
+    maxima = torch.arange(n) + base
     elems = (torch.arange(-9 * n, n) + base).to(torch.int16)
     elems = torch.cat([elems, elems | torch.tensor(-32768, dtype=torch.int16)])
     rows = []
@@ -183,6 +184,12 @@ def test_quant_rows_every_mantissa_pair(oracle, cuda, dtype):
         keep = torch.where((elems & 0x7FFF) <= a, elems, torch.zeros_like(elems))
         keep[0] = a
         rows.append(keep)
+    if bf:
+        floor = int(torch.tensor(1e-8).bfloat16().view(torch.int16)) - 1   # the largest below 1e-8, and nine binades
+        low = torch.arange(floor - 9 * n, floor + 1).to(torch.int16)
+        low = torch.cat([low, low | torch.tensor(-32768, dtype=torch.int16)])
+        assert float(low[9 * n].view(dtype)) <= 1e-8
+        rows.append(torch.nn.functional.pad(low, (0, elems.numel() - low.numel())))
     x = torch.stack(rows).view(dtype)
     x = torch.nn.functional.pad(x, (0, (-x.shape[1]) % 64))
     for r0 in range(0, x.shape[0], 64):

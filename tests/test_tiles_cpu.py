@@ -5,20 +5,10 @@ import subprocess
 
 import pytest
 
+from dispatch_rules import whole_tiles
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "pyraquant_amd", "csrc")
-
-
-def whole_tiles(tiles, K, wgx=32):
-    """Lengths of an XCD's lists, shorter and longer (the same where tiles % 8 == 0), and of each the tiles that go out whole."""
-    lengths = (tiles // 8, tiles // 8 + (1 if tiles % 8 else 0))
-    past = max(n % wgx for n in lengths)
-    rounds = tiles // 8 // wgx
-    if K >= 4096:
-        quarters = past <= wgx // 4
-    else:
-        quarters = rounds <= 4 and (past < wgx / 4 if K >= 2048 else past <= wgx / 6)
-    return lengths, tuple(n - n % wgx if quarters else n for n in lengths)
 
 
 @pytest.fixture(scope="module")

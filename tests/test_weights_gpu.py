@@ -177,21 +177,25 @@ def test_load_method_weights_package(cuda, tmp_path):
     assert rel < 2e-2, rel
 
 
-@pytest.mark.parametrize("M,lowrank", [(300, 0), (300, 32), (2100, 32), (4352, 32), (65792, 32)])
-def test_split_linear_accumulates_in_epilogue(oracle, cuda, M, lowrank):
+@pytest.mark.parametrize("M,lowrank,block", [(300, 0, "split K, 64 x 64"), (300, 32, "split K, 64 x 64"), (600, 32, "128 x 64"),
+                                             (2100, 32, "128 x 256"), (4352, 32, "256 x 256"), (6000, 32, "128 x 128"),
+                                             (65792, 32, "256 x 256")])
+def test_split_linear_accumulates_in_epilogue(oracle, cuda, M, lowrank, block):
     """The FLUX single-block proj_out split along its input (K = 3072 + 12288 -> N = 3072), both halves Int8Linear:
     the second half adds its result into the first half's output inside its GEMM epilogue (PQ_ACCUMULATE). That is
     bit-identical to torch's y0 + y1 of the two halves' outputs; without a low-rank branch it is bit-identical to the
     oracle's two layers summed with one 16-bit rounding (round(round(y0) + round(y1))), and with one it is within
-    the tolerance of the oracle's fp32 sum, on 104 sampled rows (the last 40 included) at every M: 300 runs 128 x 64
-    blocks, 2100 128 x 128 blocks, 4352 (FLUX 1K) one round of 256 x 256 blocks and 65792 (FLUX 4K, 4096^2 image +
-    256 text tokens) persistent 256 x 256 blocks."""
+    the tolerance of the oracle's fp32 sum, on 104 sampled rows (the last 40 included) at every M and so in every
+    block of the GEMM: 4352 is FLUX 1K (one round of 256 x 256 blocks), 65792 FLUX 4K (4096^2 image + 256 text tokens;
+    several rounds)."""
+    from dispatch_rules import channel_block
     from conftest import MAX_REL, MEAN_REL, bits, elem_violation, rel_errors
     from pyraquant_amd import int8_exec as E
     from pyraquant_amd import weights
     from pyraquant_amd.workloads import make_linear, make_x
 
     K0, K1, N = 3072, 12288, 3072
+    assert channel_block(M, N) == block
     lin = make_linear(K0 + K1, N, 0, True, seed=21).to(torch.bfloat16)
     split = weights.SplitInLinear(lin.to(cuda), K0)
     heads = [make_linear(k, N, lowrank, False, seed=30 + h) for h, k in enumerate((K0, K1))]
