@@ -174,11 +174,12 @@ int pq_int8_gemm_i32(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw,
  * t = x[rows] @ L1 (as pq_lowrank_down) from one pass over x: the two steps of Int8Linear.forward that read x,
  * `t = x2.to(lr_A.dtype) @ lr_A` and `quant_rows(x2)` (deploy/int8_exec.py:390-391). qp / s are bit-identical to
  * pq_quant_rows_packed; t is the fp32-accumulated product rounded to the 16-bit type, as pq_lowrank_down (the
- * accumulation order differs, so the last bit of t may differ from it). x is read from HBM once when R == 32, rows
- * are 16-byte aligned (ldx % 8 == 0) and K is one of 1024, 1280, 2048, 2560, 3072 (rows staged through LDS; every x
- * byte offset must fit 30 bits) or 4096, 6144, 8192, 10240, 12288, 15360 (rows held in registers; for K >= 8192 up to
- * 1024 rows past the last whole round of 4096, or 2048 at K = 15360, are read twice, by two kernels that spread them over
- * the chip); other shapes run the two kernels. l1t [R, K] contiguous, same dtype as x; t [M, R] with row stride ldt.
+ * accumulation order differs, so the last bit of t may differ from it; for K >= 8192 the rows read twice, below, add
+ * in an order of their own, so the last bit of a row's t may also differ between calls of different M). x is read from
+ * HBM once when R == 32, rows are 16-byte aligned (ldx % 8 == 0) and K is one of 1024, 1280, 2048, 2560, 3072 (rows
+ * staged through LDS; every x byte offset must fit 30 bits) or 4096, 6144, 8192, 10240, 12288, 15360 (rows held in
+ * registers; for K >= 8192 up to 1024 rows past the last whole round of 4096, or 2048 at K = 15360, are read twice, by
+ * two kernels that spread them over the chip); other shapes run the two kernels. l1t [R, K] contiguous, same dtype as x; t [M, R] with row stride ldt.
  * l1f: NULL, or the same matrix in the one-pass kernel's fragment order (pq_pack_lowrank_l1t, 16-byte aligned),
  * which that kernel then reads instead of l1t (contiguous 1 KB register loads: 15.8 -> 12.8 us at M = 4096,
  * K = 3072); results are identical either way, and l1t is still required (the other paths read it).
@@ -231,8 +232,9 @@ int64_t pq_int8_linear_workspace_size(int64_t M, int64_t K, int64_t R);
  * weights [N, K]; s_w [N] (group 0) or [K/32, N] (group 32); bias [N] fp32 or NULL; l1t [R, K] and l2t [N, Re] in
  * x's dtype (R a multiple of 32 up to 128, Re in {16, 32, 64} and Re <= R: the first Re columns of t enter the
  * epilogue), or NULL with R = Re = 0; l1f NULL or l1t in fragment order (as pq_quant_rows_lowrank); y [M, N] in
- * x's dtype with row stride ldy, which may overlap x. Same results as the two calls. Small layers (R == 0, group 0, K <= 4096
- * and at most 320 blocks of 16 rows x 64 outputs, past K = 2048 at most one per compute unit) run as one kernel and leave the workspace as it is. The workspace also holds the GEMM's scheduling
+ * x's dtype with row stride ldy, which may overlap x. Same results as the two calls. Small layers (R == 0, group 0,
+ * K <= 4096 and at most 320 blocks of 16 rows x 64 outputs, past K = 2048 at most one per compute unit; y apart from x)
+ * run as one kernel and leave the workspace as it is. The workspace also holds the GEMM's scheduling
  * buffer (pq_int8_gemm's sched), which the quantizer kernel zeroes, so a large layer claims its blocks even when
  * replayed from a graph; calls that may overlap need workspaces of their own.
  * Replaces the body of `Int8Linear.forward` (deploy/int8_exec.py:382-393): one C call per layer.

@@ -1206,8 +1206,8 @@ inline int64_t small_blocks(const GemmArgs& a) { return (int64_t)((a.M + 127) / 
 //   4x its work, so one round of them beats the extra round of small blocks. Measured at M = 4352 (FLUX's 1K token
 //   count), bit-identical outputs: 56.7 -> 45.2 us at K = N = 3072, 182 -> 150 us at K = 12288, N = 3072, 226 ->
 //   179 us at K = 15360; at M = 4096, K = N = 3072: 46.0 -> 44.4 us. Where the 128 x 128 blocks fit in one round
-//   (M = 2048) or the 256 x 256 ones need a second (M = 8192), 128 x 128 stays faster (27.7 against 35.9 us, 92
-//   against 94.6 us).
+//   (M = 2048) or the 256 x 256 ones need a second (M = 8192) smaller blocks stay faster: 128 x 128 27.7 against 35.9 us
+//   (and 128 x 256 24 us, see dispatch_tiles), 92 against 94.6 us.
 inline bool big_tiles(const GemmArgs& a, hipStream_t stream) {
   const int64_t tiles = (int64_t)((a.M + 127) / 128) * ((a.N + 255) / 256);
   if (tiles >= 1024) return true;
@@ -1261,13 +1261,13 @@ int dispatch_tiles(GemmArgs& a, hipStream_t stream) {
     if (big_tiles(a, stream)) return launch_dma<4, 2, 4, 1, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     // More 128 x 128 blocks than CUs, but blocks twice as tall (8 waves, the ping-pong loop) all fit at once: one
     // of them takes less than the two blocks it replaces do sharing a CU. M x K x N, 128 x 128 and 128 x 256: 2048 x 3072 x
-    // 3072 29.1 and 24.4 us, 512 x 3072 x 12288 28.9 and 24.8, 4096 x 2560 x 1280 22.1 and 20.0, 4096 x 640 x 1280 11.0
-    // and 10.0. With one 128 x 128 block per CU or less they lose (2048 x 3072 x 2048 17.8 and 22.0), and in a second round
+    // 3072 26.6 and 23.8 us, 512 x 3072 x 12288 26.8 and 23.9, 4096 x 2560 x 1280 22.1 and 19.3, 4096 x 640 x 1280 10.0
+    // and 9.5. With one 128 x 128 block per CU or less they lose (2048 x 3072 x 2048 17.8 and 22.0), and in a second round
     // (2700 x 3072 x 3072 35.9 and 44.2).
     const int64_t wgs = persistent_workgroups(stream);
     if (small_blocks(a) > wgs && (int64_t)((a.M + 255) / 256) * ((a.N + 127) / 128) <= wgs)
       return launch_dma<2, 2, 4, 1, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
-    // fewer 128 x 128 blocks than half the CUs: 128 x 64 blocks (measured 1.3x faster at 80 blocks, even at 160)
+    // fewer 128 x 128 blocks than half of 256 CUs: 128 x 64 blocks (measured 1.3x faster at 80 blocks, even at 160)
     if (small_blocks(a) < 128) return launch_dma<2, 1, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
     return launch_dma<2, 2, 2, 2, PACKED, MODE, LRS, LRDT, ODT, ACC>(a, stream);
   }

@@ -10,8 +10,8 @@
 //
 // Exact codes without one IEEE division per element and without a branch: with c = fl(1/s),
 //   q0 = fl(x c); r = fma(-q0, s, x) (the remainder of q0, exact); q = fma(r, c, q0)
-// is the Newton step that ends a correctly rounded division, and rint(q) == rint(fl(x / s)) for every row maximum a and
-// every |x| <= a of both 16-bit types: the result depends on the two mantissas and the exponent difference alone, and
+// is the Newton step that ends a correctly rounded division (P. Markstein, IBM J. Res. Dev. 34 (1990), 111-119), and
+// rint(q) == rint(fl(x / s)) for every row maximum a and every |x| <= a of both 16-bit types: the result depends on the two mantissas and the exponent difference alone, and
 // all of those pairs (and the floor s = fl(1e-8) / 127) have been compared. q + 1.5 * 2^23 holds the rounded code in its
 // low byte (round to nearest even; |q| < 2^22). Four instructions per element. A test for near ties with the division
 // beside it was as many, and its code, repeated for every chunk of a row, was what bound the kernels: 1.7 KB per
@@ -898,7 +898,8 @@ constexpr int kWideWaves = 8;                 // waves per workgroup, two rows e
 constexpr int kWideSlab = 512;                // K elements per slab
 constexpr int kWidePitch = 2 * kWideSlab + 16;   // LDS row pitch: consecutive rows 16 bytes apart in the bank window
 constexpr int kWideRedPitch = 36;             // floats per row of the partial-sum buffer
-constexpr int kWideGrid = 256;                // workgroups, one per CU
+constexpr int kWideGrid = 256;                // workgroups, one per CU of the 256 it was measured on (a part with fewer
+                                              // runs them in turn)
 constexpr int64_t kTailRows = 1024;           // rows past whole rounds that take the partial-sum kernel instead
 
 template <int DT, int NCH, int RPW>   // NCH = K / 512: 16-byte chunks per lane per row, and slabs; RPW rows per wave
@@ -1185,7 +1186,7 @@ constexpr int kSmallMaxK = 4096;   // 64 KB of codes
 // the CUs take a second round. One kernel and two, replayed from a graph over eight layers: at K = 2112, 128 x 2048 (256
 // workgroups) 7.4 and 9.9 us, 96 x 3072 (288) 12.8 and 10.0; at K = 3072 the same rows 8.6 and 10.8, 15.1 and 10.8; at K =
 // 4096, 256 x 1024 (256) 9.4 and 12.9, 77 x 4096 (320) 16.9 and 12.2, 16 x 20480 (320) 26.1 and 24.0. At K = 2048 two fit:
-// 96 x 3072 (288) 8.6 and 9.4, 77 x 4096 (320) 8.6 and 9.3.
+// 96 x 3072 (288) 8.6 and 9.4, 77 x 4096 (320) 8.6 and 9.3. (Measured on 256 CUs; the 320 is theirs.)
 constexpr int64_t kSmallBlocks = 320;
 constexpr int64_t kSmallTwoPerCuK = 2048;
 

@@ -2,9 +2,9 @@
 
 The reference needs a second Triton autotune set for N % 256 != 0 (N = 640) and a direct-launch cache
 ("FAST_LAUNCH") to bring the per-call Python overhead from 75/100 us down to 8/11 us
-(deploy/run_sdxl_latency.py:143-195). Here both are native: the HIP GEMM takes any N % 64 == 0 and every
-call is one ctypes call into the C ABI, with no JIT or autotune dispatch. ``FAST_LAUNCH`` is kept as a flag
-for driver compatibility; it changes nothing.
+(deploy/run_sdxl_latency.py:143-195). Here both are native: the HIP GEMM takes any N % 64 == 0 and every layer
+call is one call into the library (through _direct.so without a low-rank branch, by ctypes with one), with no JIT or
+autotune dispatch. ``FAST_LAUNCH`` is kept as a flag for driver compatibility; it changes nothing.
 
 Group-32 W8A8 (config 3): ``SdxlInt8Linear(lin, group_size=32)`` keeps one fp32 scale per 32 consecutive K
 elements per output channel (pyraquant/quantizers_weight.py:96-109) and applies it inside the MFMA K loop.
