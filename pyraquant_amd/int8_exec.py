@@ -391,7 +391,8 @@ def _convert_weight(w: torch.Tensor, group_size: int, pack: bool):
     wk = w.detach()
     if wk.dtype not in _WEIGHT_DTYPES or type(wk) is not torch.Tensor:   # (a subclass says itself what its values are)
         wk = wk.float()
-    wk = wk.resolve_neg()
+    if wk.is_neg():
+        wk = wk.resolve_neg()
     N, K = wk.shape
     # the kernels read a 16-bit weight in place: dense, where its elements or its rows are not (an expanded row, windows)
     if wk.stride(1) != 1 or (wk.dtype != torch.float32 and wk.stride(0) < K):
@@ -632,9 +633,10 @@ class Int8Linear(nn.Module):
         if accumulate:
             assert out is not None, "accumulate=True adds into out="
         if row_idx is None and out is None and out_row_idx is None and DIRECT_CALLS:
-            d, b = self.__dict__, self._buffers
-            if d.get("lr_A", d) is None and d.get("weight_packed", b.get("weight_packed")) is not None:
-                y = (_direct_linear or _load_direct())(d, b, x)   # no low-rank branch: native
+            d = self.__dict__
+            # no low-rank branch: native (loaded for the first layer that it can take)
+            if _direct_linear is not None or (d.get("lr_A", d) is None and self.weight_packed is not None):
+                y = (_direct_linear or _load_direct())(d, self._buffers, x)
                 if y is not None:
                     if type(y) is int:
                         _lib.check(y, "int8_linear")
